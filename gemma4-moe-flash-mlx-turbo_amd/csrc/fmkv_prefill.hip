@@ -7,40 +7,64 @@
 // lo(p) <= j <= p, lo(p) = max(trim, p - W + 1) on sliding layers.
 //
 // One work-group = 64 query rows (a row is one (position, q head) of the
-// KV head's GQA group: 64 / G consecutive positions) of one KV head, four
-// wave pairs of 16 rows each. All four pairs read the same staged
-// head-block, so one copy HBM -> LDS serves 64 rows. Inside a pair the two
-// waves own one half of head_dim each (half the 64-dim groups), exchange
-// their partial scores once per block through LDS (flag handshake) and run
-// identical softmax bookkeeping, as the decode kernel's pairs do; the
-// matrix-core columns are the pair's 16 rows.
+// KV head's GQA group: 64 / G consecutive positions) of one KV head; a step
+// covers 32 keys (two head-blocks). head_dim is split over the waves: wave g
+// of the D / 64 owns the 64 dims of group g for all 64 rows, in both
+// products, so every stored code is read from memory and turned into a
+// matrix-core operand by exactly one wave of the work-group, straight into
+// registers (no LDS staging), and is used for four 16-row tiles. (One pair of
+// waves per 16 rows, every pair decoding every block, took 7.78 ms for a
+// 2048-token chunk after 32768 positions, 16 q / 2 KV heads of 512 dims, 8
+// bits; this split takes 5.28 ms, and 0.148 against 0.227 ms for a 2048-token
+// chunk on a 1024-position ring, 16 / 8 heads of 256 dims, 4 bits.)
 //
-// Per block (16 keys), affine caches, per 64-dim group g of the wave's half:
-//   QK^T  S^T[16 key x 16 row] += K[16 x 32] . Q^T[32 x 16] with K codes as
-//         exact f16 integers, q_rot as an f16 high part and an f16 residual
-//         (~22 bits), the residual's products first, then the high part's,
-//         in one accumulator; then s += scale * acc + bias * sum(q_group). (The decode
-//         kernel's 1024 + code operands, one v_perm per two codes, left the
-//         residual's contribution on top of a large partial sum here: the
-//         worst output error of a 1500-key test rose ~4x; the plain codes
-//         cost one packed subtract more per two codes.)
-//   PV    O^T[16 dim x 16 row] += V^T[16 dim x 16 key] . P'^T[16 key x 16 row]
-//         with P' = p * v_scale as f16 high part + residual (two MFMAs);
-//         the bias terms are summed on the side.
-// Codebook (TurboQuant) caches, per 32-dim slice / 16-dim tile of the
-// wave's half: the indices become f16 centroid operands through the decode
-// kernel's LDS lookup table (fmkv_cb_common.h). 2 and 3 bits: the exact
-// integer operands 1000 * centroid, S^T = C . q_hi + C . q_lo, scaled per
-// key by norm / (1000 sqrt(D)); O^T likewise with P' = p * norm /
+// What bounds it: the issue of matrix and vector instructions together. A
+// 16x16x32 MFMA alone takes 8.7 ns of a SIMD, with four independent FMAs after
+// it 12.4 ns (the FMAs alone: 5): they hardly overlap, also between the two
+// waves of a SIMD. Of the 2.5 us of a step of a SIMD (8 bits, head_dim 512)
+// its 128 MFMAs are 1.1 us, the conversion of codes and weights, the scales
+// and the softmax the rest. Hence the packed f16 arithmetic on the weights
+// (v_pk_* 1.9 ns for two elements; v_fma_mixlo_f16 3.7 ns for one).
+//
+//   QK^T  S_g^T[32 key x 64 row] = K_g . Q_g^T per wave: a partial score over
+//         its 64 dims, handed through LDS to the wave that sums the row's
+//         partials;
+//   softmax of 64 / (D / 64) rows per wave: sum, mask, running max, weights
+//         P to LDS, and the factor by which every wave rescales its row
+//         accumulators when a row's reference max moved;
+//   PV    O_g^T[64 dim x 64 row] += V_g^T[64 dim x 32 key] . P^T[32 key x 64
+//         row] per wave.
+//
+// The three stages run as a pipeline, one barrier per step: between two
+// barriers a wave issues the QK of step i + 1, the softmax of step i and the
+// PV of step i - 1, which depend on nothing of one another (score and weight
+// buffers alternate), so the two waves of a SIMD overlap one's matrix-core
+// work with the other's vector work. Codes are loaded a step ahead.
+//
+// Operands, affine caches: K and V codes as exact f16 integers, q_rot as an
+// f16 high part and an f16 residual (~22 bits), the residual's products
+// first, then the high part's, in one accumulator; then s_g = scale * acc +
+// bias * sum(q_group); P' = p * v_scale likewise as f16 high part and residual
+// (two MFMAs), the bias terms summed on the side in f32. (Codes as f16
+// subnormals, code * 2^-24, would save the subtract of the conversion, but
+// the matrix cores keep 2 bits less of such products: relative error 1.7e-7
+// against 5e-8 over 32 products.)
+// Codebook (TurboQuant) caches: the indices become f16 centroid operands
+// through the decode kernel's LDS lookup table (fmkv_cb_common.h). 2 and 3
+// bits: the exact integer operands 1000 * centroid, S^T = C . q_lo + C . q_hi,
+// scaled per key by norm / (1000 sqrt(D)); O^T likewise with P' = p * norm /
 // (1000 sqrt(D)) as f16 high part and residual (two MFMAs each). 4 bits: the
 // centroids' f16 high part and residual, S^T = C_hi . q_hi + C_lo . q_hi +
 // C_hi . q_lo and O^T likewise (three MFMAs each: the fourth product is below
 // f32 rounding).
 // Plain (bf16) caches read K rows and V columns as bf16 operands
-// (v_mfma_f32_16x16x32_bf16 / 16x16x16_bf16) against the raw bf16 q (exact
-// products; the softmax scale applies after), P as bf16 high part and
-// residual; no rotation.
-// Blocks wholly outside a pair's rows' windows are skipped by that pair.
+// (v_mfma_f32_16x16x32_bf16) against the raw bf16 q (exact products; the
+// softmax scale applies after), P as bf16 high part and residual; no rotation.
+//
+// The 32 keys of a PV product are ordered [4j .. 4j+3 of the first block,
+// 4j .. 4j+3 of the second] for lane group j on both operands: V codes as
+// stored for one block's 16-key tile feed the 32-key instruction, which has
+// twice the 16-key one's rate.
 //
 // A paged pool runs one sequence per grid z with its own start position and
 // block table (linear sequences: the append goes first).
@@ -50,12 +74,6 @@
 // positions early queries still need), the rest from new_st (a staging
 // copy of the chunk, or the cache itself for linear caches). A block that
 // straddles p_split is visited once per store with the other part masked.
-//
-// Copies: each wave issues CP copy instructions per block (the block's
-// codes and scale/bias, zero-padded past their end) into one of NST stages;
-// a block is used after every wave waited for its own copies and a
-// work-group barrier; the next block's copies are then issued into the
-// stage the previous block freed.
 #include "fmkv_device.h"
 #include "fmkv_internal.h"
 #include "fmkv_attn_common.h"
@@ -64,26 +82,30 @@
 namespace fmkv {
 namespace {
 
-constexpr int kPfWaves = 8;   // four pairs
-constexpr int kPfRows = 64;   // query rows per work-group (16 per pair)
-constexpr int kPfStages = 3;
+constexpr int kPfRows = 64;   // query rows per work-group, four matrix-core tiles
+constexpr int kPfTiles = kPfRows / 16;
+constexpr int kPfKeys = 2 * kBlockTokens;  // keys per step
+constexpr int kPfQuads = kPfKeys / 4;      // groups of four keys of a step
 
 template <int D, int BITS, int MODE>
 struct PfPlan {
   static constexpr BlockLayout L = make_layout(D, BITS, MODE);
   static constexpr int NG = D / 64;
-  static constexpr int GH = NG / 2;  // groups per wave
-  static constexpr int NSW = D / 64;  // 32-dim QK slices per wave
-  static constexpr int NTW = D / 32;  // 16-dim PV tiles per wave
-  // the bytes of a head-block the kernel reads: affine [K codes][V codes]
-  // [K meta][V meta]; codebook [K codes][V codes][K norms, padded][V norms];
-  // plain [K rows][V columns]
-  static constexpr int kBytes = MODE == kAffine     ? (int)(2 * L.code_bytes) + 2 * NG * 64
-                                : MODE == kCodebook ? (int)L.v_meta + 2 * kBlockTokens
-                                                    : (int)(2 * L.code_bytes);
-  static constexpr int kNC = (kBytes + kChunk - 1) / kChunk;
-  static constexpr int CP = (kNC + kPfWaves - 1) / kPfWaves;  // copies per wave per block
-  static constexpr int kStageBytes = kPfWaves * CP * kChunk;
+  static constexpr int NW = NG;  // waves: one per 64 dims
+  // The softmax stage: with 8 waves a wave sums 8 rows, lane l holding key
+  // quad l >> 3 of row l & 7. With 4 (2) waves it sums one (two) whole row
+  // tiles in the QK accumulators' own layout, so its own partial stays in
+  // registers.
+  static constexpr bool kOwn = NW < 8;
+  static constexpr int NRS = NW == 2 ? 2 : 1;  // row sets per lane
+  static constexpr int NQ = kOwn ? 2 : 1;      // key quads per lane and row set
+  static constexpr int kSrc = kOwn ? NW - 1 : NW;  // partials of a tile in LDS
+  static constexpr int kXs = kPfTiles * kSrc * 2 * 1024;  // one score buffer
+  static constexpr int kPb = kPfQuads * kPfRows * 16;     // one weight buffer
+  static constexpr int kPbOff = 2 * kXs;
+  static constexpr int kAlOff = kPbOff + 2 * kPb;
+  static constexpr int kLutOff = kAlOff + 2 * kPfRows * 4;
+  static constexpr int kLutBytes = MODE == kCodebook ? CbLut<BITS == 16 ? 2 : BITS>::kBytes : 0;
   static constexpr int kQStride = D + 8;  // 16-bit values per q-table row (padding against bank conflicts)
   // q table: high and residual parts of q_rot (affine: and group sums);
   // plain: the raw bf16 rows
@@ -91,69 +113,88 @@ struct PfPlan {
                                (MODE == kAffine ? kPfRows * NG * 4 : 0);
   static constexpr int kRStride = D + 4;  // f32 per output row
   static constexpr int kRows = kPfRows * kRStride * 4;
-  // codebook: the centroid lookup table follows the stages
-  static constexpr int kLutOff = kPfStages * kStageBytes;
-  static constexpr int kLutBytes = MODE == kCodebook ? CbLut<BITS == 16 ? 2 : BITS>::kBytes : 0;
   static constexpr int kRegion = cmax(cmax(kLutOff + kLutBytes, kQTab), kRows);
-  static_assert(MODE != kAffine || ((int)L.k_meta == (int)(2 * L.code_bytes) &&
-                                    (int)L.v_meta == (int)L.k_meta + NG * 64),
-                "codes and scale/bias are contiguous in a head-block");
-  static_assert(kPfStages * CP <= 63, "vmcnt immediates");
+  // words per lane of one block's codes of the wave's 64 dims
+  static constexpr int KW = MODE == kAffine ? BITS / 2 : MODE == kPlain ? 8 : BITS == 3 ? 4 : 2;
+  static constexpr int VW = MODE == kAffine ? BITS / 2 : MODE == kPlain ? 8 : BITS == 3 ? 8 : 4;
 };
 
-// K operand of MFMA s of group g as the plain codes (exact f16 integers).
+// K operand of MFMA s of group g as the plain codes (exact f16 integers);
+// w: the lane's words of the group.
 template <int BITS>
-__device__ inline half8_t k_operand_plain(const u32x4 w, int g, int s) {
+__device__ inline half8_t k_operand_plain(const uint32_t* w, int s) {
   if constexpr (BITS == 8) {
     const uint32_t w0 = w[2 * s], w1 = w[2 * s + 1];
     return cat8(u8x2_to_h2(w0, 0x04010400u), u8x2_to_h2(w0, 0x04030402u),
                 u8x2_to_h2(w1, 0x04010400u), u8x2_to_h2(w1, 0x04030402u));
   } else {
-    return k_operand<BITS>(w, g, s);
+    return cat8(u4x2_to_h2(w[s], 0), u4x2_to_h2(w[s], 1), u4x2_to_h2(w[s], 2), u4x2_to_h2(w[s], 3));
+  }
+}
+
+// V operand of column tile ct: tokens 4j .. 4j+3 of two blocks, as the plain
+// codes; wa, wb: the lane's words of the group in either block.
+template <int BITS>
+__device__ inline half8_t v_operand_plain(const uint32_t* wa, const uint32_t* wb, int ct) {
+  if constexpr (BITS == 8) {
+    return cat8(u8x2_to_h2(wa[ct], 0x04010400u), u8x2_to_h2(wa[ct], 0x04030402u),
+                u8x2_to_h2(wb[ct], 0x04010400u), u8x2_to_h2(wb[ct], 0x04030402u));
+  } else {
+    const int k0 = (ct & 1) * 2;
+    return cat8(u4x2_to_h2(wa[ct >> 1], k0), u4x2_to_h2(wa[ct >> 1], k0 + 1),
+                u4x2_to_h2(wb[ct >> 1], k0), u4x2_to_h2(wb[ct >> 1], k0 + 1));
   }
 }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef short short4_t __attribute__((ext_vector_type(4)));
-
 __device__ inline uint32_t pack_bf16x2(float a, float b) {
   return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
 }
 
+// A uniform address in memory and loads at a lane's offset from it. (Global
+// address space: a generic pointer's flat loads also count as LDS operations,
+// and every wait for LDS data or at a barrier would wait for memory too.)
+typedef const uint8_t __attribute__((address_space(1)))* gptr_t;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_a4 __attribute__((aligned(4)));  // two words at a 4-byte boundary
+template <class T>
+__device__ inline T load_at(gptr_t p, uint32_t off) {
+  return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off);
+}
+
+// LDS of this wave written, every wave of the work-group here. Loads from
+// memory stay in flight across it.
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 template <int D, int BITS, int MODE>
-__global__ __launch_bounds__(kPfWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(D)  // a wave per 64 dims
+__attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_attn_kernel(PrefillArgs a) {
   using P = PfPlan<D, BITS, MODE>;
   constexpr BlockLayout L = P::L;
-  constexpr int NG = P::NG, GH = P::GH, E = D / 64, LPG = 64 / E;
-  constexpr int NSW = P::NSW, NTW = P::NTW;
-  constexpr int CP = P::CP, NST = kPfStages, SB = P::kStageBytes;
+  constexpr int NG = P::NG, NW = P::NW, E = D / 64, LPG = 64 / E;
+  constexpr int NRS = P::NRS, NQ = P::NQ, KW = P::KW, VW = P::VW;
+  constexpr bool kOwn = P::kOwn;
   constexpr int QS = P::kQStride, RS = P::kRStride;
   // codebook index width (the template's BITS; other modes never use it)
   constexpr int CB = MODE == kCodebook ? BITS : 2;
 
   __shared__ __align__(16) uint8_t region[P::kRegion];
-  __shared__ __align__(16) float4_t xs[kPfWaves * 2 * 64];
-  __shared__ int xflag[kPfWaves];
   __shared__ float lrow[kPfRows];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pair = wave >> 1, half = wave & 1;
   const int j = lane >> 4, c = lane & 15;
-  const int g0 = half * GH;
   const int G = a.group;
   const int QP = kPfRows / G;  // query positions per work-group
   const int kvh = blockIdx.y, seq = blockIdx.z;
   const int qi0 = blockIdx.x * QP;
-  // per-sequence start and block table (paged) through scalar loads, which
-  // never wait for the copies in flight
+  // paged: the sequence's start, through a scalar load (everything derived
+  // from it stays in scalar registers)
   typedef const int32_t __attribute__((address_space(4)))* cint_ptr;
   const int64_t p0 = a.start_pos ? (int64_t)((cint_ptr)(uintptr_t)a.start_pos)[seq] : a.p0;
-  const cint_ptr table =
-      a.new_st.block_table
-          ? (cint_ptr)(uintptr_t)(a.new_st.block_table + (int64_t)seq * a.new_st.table_stride)
-          : nullptr;
   const int nq = a.n_q - qi0 < QP ? a.n_q - qi0 : QP;  // valid positions of the tile
 
   // visible keys of position p: [lo(p), p]
@@ -162,24 +203,11 @@ void prefill_attn_kernel(PrefillArgs a) {
     if (a.window > 0 && p - a.window + 1 > lo) lo = p - a.window + 1;
     return lo < 0 ? 0 : lo;
   };
-  // this lane's row = column c of its pair
-  const int row = pair * 16 + c;
-  const int rq = row / G;
-  const bool row_valid = rq < nq;
-  const int64_t p_row = p0 + qi0 + rq;
-  const int64_t row_lo = lo_of(p_row);
-  // the pair's positions [pA, pB] (pair-uniform)
-  const int pq0 = (pair * 16) / G;
-  int pq1 = (pair * 16 + 15) / G;
-  if (pq1 > nq - 1) pq1 = nq - 1;
-  const bool pair_any = pq0 <= pq1;
-  const int64_t pA = p0 + qi0 + pq0, pB = p0 + qi0 + pq1;
-  const int64_t pair_lo_min = lo_of(pA), pair_lo_max = lo_of(pB);
-  const bool pair_full_rows = (pair * 16 + 15) / G < nq;  // all 16 rows are real queries
 
   // ---- virtual blocks of the work-group: [lo(first), last] in 16-key
   // blocks, the part below p_split from old_st, the rest from new_st ----
-  const int64_t wg_lo = lo_of(p0 + qi0), wg_hi = p0 + qi0 + nq - 1;
+  const int64_t pA = p0 + qi0, pB = p0 + qi0 + nq - 1;
+  const int64_t wg_lo = lo_of(pA), wg_hi = pB;
   const int64_t b_lo = wg_lo / kBlockTokens, b_hi = wg_hi / kBlockTokens;
   const int64_t ps = a.p_split;
   int64_t old_last = (ps + kBlockTokens - 1) / kBlockTokens - 1;  // last block with keys < ps
@@ -189,92 +217,87 @@ void prefill_attn_kernel(PrefillArgs a) {
   if (new_first < b_lo) new_first = b_lo;
   const int64_t n_new = b_hi >= new_first ? b_hi - new_first + 1 : 0;
   const int nvb = (int)(n_old + n_new);
-  // Per-block tests in 32-bit scalar form (the scalar unit has no 64-bit
-  // signed compares, and the vector unit's would cost every block): block
-  // rb = b - b_lo. A block that p_split cuts (cut_rb, visited once per
-  // store with its own part) takes the 64-bit tests; any other holds keys
-  // t0 .. t0 + 15, so the pair sees it when sees_lo <= rb <= sees_hi (a key
-  // at or past the pair's smallest lower bound, one at or before its last
-  // position) and it is whole for every row of the pair when full_lo <= rb
-  // <= full_hi (every key at or past the largest lower bound, at or before
-  // the first position). (When the pair has rows, its bounds are at or past
-  // b_lo's first key.)
+  const int nst = (nvb + 1) / 2;  // steps of two virtual blocks
+  // Positions below are 32-bit and relative to the first block's first key
+  // (a cache holds less than 2^31 positions). Virtual block i holds keys
+  // 16 rb .. of block rb = i (old store) or i + vb_shift, of which those in
+  // [vlo, vhi) are its own; past the last one the range is empty.
   const int64_t bl16 = b_lo * kBlockTokens;
-  auto rel_blk = [&](int64_t x) -> int {  // floor(x / 16) for x >= 0, clamped; -1 below
-    if (x < 0) return -1;
-    const int64_t q = x / kBlockTokens;
-    return (int)(q < INT32_MAX - 1 ? q : INT32_MAX - 1);
+  auto rel = [&](int64_t x) __attribute__((always_inline)) -> int {
+    x -= bl16;
+    return (int)(x < -(1 << 30) ? -(1 << 30) : x > INT32_MAX ? INT32_MAX : x);
   };
-  const int sees_lo = pair_any ? rel_blk(pair_lo_min - bl16) : INT32_MAX;
-  const int sees_hi = pair_any ? rel_blk(pB - bl16) : -1;
-  const int full_lo = pair_any && pair_full_rows ? rel_blk(pair_lo_max - bl16 + kBlockTokens - 1)
-                                                  : INT32_MAX;
-  const int full_hi = pair_any ? rel_blk(pA - (kBlockTokens - 1) - bl16) : -1;
-  const int cut_rb = ps % kBlockTokens != 0 ? rel_blk(ps - bl16) : -1;
-  const int new_rb0 = (int)(new_first - b_lo);  // rb of virtual block n_old
-  // virtual block i's absolute block and valid key range [vlo, vhi)
-  struct VB {
-    int64_t b, vlo, vhi;
+  const int b_lo_i = (int)b_lo, n_old_i = (int)n_old, vb_shift = (int)(new_first - b_lo) - n_old_i;
+  const int ps_r = rel(ps), vis_r = rel(lo_of(0)), pA_r = rel(pA);
+  const int win = (int)(a.window < INT32_MAX ? a.window : INT32_MAX);
+  auto lo_rel = [&](int p) __attribute__((always_inline)) -> int {  // lo(p), relative
+    return win > 0 && p - win + 1 > vis_r ? p - win + 1 : vis_r;
   };
-  auto vb_of = [&](int i) -> VB {
-    VB v;
-    if (i < n_old) {
-      v.b = b_lo + i;
-      v.vlo = v.b * kBlockTokens;
-      v.vhi = (v.b + 1) * kBlockTokens < ps ? (v.b + 1) * kBlockTokens : ps;
-    } else {
-      v.b = new_first + (i - n_old);
-      v.vlo = v.b * kBlockTokens > ps ? v.b * kBlockTokens : ps;
-      v.vhi = (v.b + 1) * kBlockTokens;
-    }
-    return v;
+  auto vb_range = [&](int i, int& vlo, int& vhi) __attribute__((always_inline)) {
+    const bool old = i < n_old_i;
+    const int t0 = (old ? i : i + vb_shift) * kBlockTokens, t1 = t0 + kBlockTokens;
+    vlo = old ? t0 : t0 > ps_r ? t0 : ps_r;
+    vhi = old ? (t1 < ps_r ? t1 : ps_r) : i < nvb ? t1 : vlo;
   };
-  // its head-block. A ring's slot block of virtual block i is ring0 + i
+  // Virtual block i's head-block (past the last one: the last one's), in
+  // scalar arithmetic. A ring's slot block of virtual block i is ring0 + i
   // modulo its nrb blocks (the old keys lie in the last W positions before
   // p_split: n_old <= nrb + 1, so two conditional subtractions reduce it).
   const int nrb = a.ring_slots > 0 ? (int)(a.ring_slots / kBlockTokens) : 0;
   const int ring0 = nrb > 0 ? (int)(b_lo % nrb) : 0;
   const int32_t n_pool = (int32_t)(a.new_st.n_blocks < INT32_MAX ? a.new_st.n_blocks : INT32_MAX);
-  auto blk_ptr = [&](int i) -> const uint8_t* {
-    if (i < n_old) {
-      int64_t phys = b_lo + i;
+  const uint64_t base_old = reinterpret_cast<uint64_t>(a.old_st.base) + kvh * a.old_st.head_stride;
+  const uint64_t base_new = reinterpret_cast<uint64_t>(a.new_st.base) + kvh * a.new_st.head_stride;
+  const uint32_t t_width = a.new_st.block_table ? (uint32_t)a.new_st.table_stride : 0;
+  const cint_ptr table =
+      (cint_ptr)(uintptr_t)(a.new_st.block_table + (int64_t)seq * a.new_st.table_stride);
+  auto blk_ptr = [&](int i) __attribute__((always_inline)) -> gptr_t {
+    i = i < nvb ? i : nvb - 1;
+    if (i < n_old_i) {
+      uint32_t phys = (uint32_t)(b_lo_i + i);
       if (nrb > 0) {
         int r = ring0 + i;
         r -= r >= nrb ? nrb : 0;
         r -= r >= nrb ? nrb : 0;
-        phys = r;
+        phys = (uint32_t)r;
       }
-      return a.old_st.base + phys * a.old_st.block_stride + (int64_t)kvh * a.old_st.head_stride;
+      return (gptr_t)(base_old + (uint64_t)phys * (uint64_t)a.old_st.block_stride);
     }
-    const int64_t b = new_first + (i - n_old);
-    int64_t phys = b - a.new_blk0;
-    if (table) {
+    const uint32_t b = (uint32_t)(b_lo_i + i + vb_shift);
+    uint32_t phys = b - (uint32_t)a.new_blk0;
+    if (a.new_st.block_table) {
       // a table entry outside the pool (or a position past the table's
       // width) reads a valid block rather than faulting
-      int32_t e = 0;
-      if ((b >> 31) == 0 && (uint32_t)b < (uint32_t)a.new_st.table_stride) e = table[(uint32_t)b];
-      phys = e < 0 ? 0 : (e >= n_pool ? n_pool - 1 : e);
+      const int32_t e = b < t_width ? table[b] : 0;
+      phys = (uint32_t)(e < 0 ? 0 : (e >= n_pool ? n_pool - 1 : e));
     }
-    return a.new_st.base + phys * a.new_st.block_stride + (int64_t)kvh * a.new_st.head_stride;
+    return (gptr_t)(base_new + (uint64_t)phys * (uint64_t)a.new_st.block_stride);
+  };
+  // every key of virtual block i is visible to every row: at or past the
+  // largest lower bound, at or before the first position, not cut by p_split
+  const int lo_max = lo_rel(pA_r + nq - 1);
+  auto blk_full = [&](int i) __attribute__((always_inline)) -> bool {
+    int vlo, vhi;
+    vb_range(i, vlo, vhi);
+    return vhi - vlo == kBlockTokens && vlo >= lo_max && vhi - 1 <= pA_r;
   };
 
-  // ---- q_rot of the 64 rows: rows wave + 8 k, high / residual halves
+  // ---- q_rot of the 64 rows: rows wave + NW k, high / residual halves
   // (plain: the raw bf16 rows) ----
   _Float16* const qhi = reinterpret_cast<_Float16*>(region);
   _Float16* const qlo = qhi + kPfRows * QS;
   float* const qsum = reinterpret_cast<float*>(qlo + kPfRows * QS);  // [row][NG] (affine)
   const uint32_t sbits = lane_sign_bits<D>(a.sign_bits, lane);
   const float cs_lane = fwht_lane_sign(lane) * a.c;
-  if (lane == 0) xflag[wave] = 0;
-#pragma unroll 1
-  for (int k = 0; k < kPfRows / kPfWaves; k++) {
-    const int r = wave + kPfWaves * k;
+#pragma unroll 2
+  for (int k = 0; k < kPfRows / NW; k++) {
+    const int r = wave + NW * k;
     const int rq_ = r / G, rh_ = r - (r / G) * G;
+    const uint16_t* const src =
+        a.q + (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D +
+        lane * E;
     if constexpr (MODE == kPlain) {
       // E consecutive bf16 of the row as stored (zero past the chunk)
-      const uint16_t* src =
-          a.q + (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D +
-          lane * E;
       uint16_t* dst = reinterpret_cast<uint16_t*>(qhi + r * QS + lane * E);
 #pragma unroll
       for (int i = 0; i < E; i++) dst[i] = rq_ < nq ? src[i] : (uint16_t)0;
@@ -284,8 +307,7 @@ void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
     for (int i = 0; i < E; i++) x[i] = 0.0f;
     if (rq_ < nq) {
-      load_row<E>(a.q + (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D +
-                      lane * E, x);
+      load_row<E>(src, x);
 #pragma unroll
       for (int i = 0; i < E; i++) x[i] = x[i] * a.qscale;
     }
@@ -308,358 +330,539 @@ void prefill_attn_kernel(PrefillArgs a) {
   }
   __syncthreads();
 
-  // this wave's B operands: its pair's 16 rows, its groups; the lane (j, c)
-  // holds 8 consecutive dims of row `row` at the K-code placement
-  // (codebook and plain: slice k = 2 gi + s of the wave's half, dims
-  // half * D / 2 + 32 k + 8 j ..; plain B operands are the bf16 bits)
-  half8_t bqh[GH][2], bql[GH][2];
-  float qs[GH];
+  // this wave's B operands: its 64 dims of every row tile; the lane (j, c)
+  // holds 8 consecutive dims of row 16 rt + c at the K-code placement
+  // (codebook and plain: slice s, dims 64 wave + 32 s + 8 j ..; plain B
+  // operands are the bf16 bits)
+  half8_t bqh[kPfTiles][2], bql[kPfTiles][2];
+  float qs[kPfTiles];
 #pragma unroll
-  for (int gi = 0; gi < GH; gi++) {
-    const int g = g0 + gi;
+  for (int rt = 0; rt < kPfTiles; rt++) {
+    const int row = rt * 16 + c;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-      const int d0 = MODE == kAffine ? g * 64 + (BITS == 8 ? j * 16 + s * 8 : s * 32 + j * 8)
-                                     : half * (D / 2) + (2 * gi + s) * 32 + j * 8;
-      bqh[gi][s] = *reinterpret_cast<const half8_t*>(qhi + row * QS + d0);
-      if constexpr (MODE != kPlain) bql[gi][s] = *reinterpret_cast<const half8_t*>(qlo + row * QS + d0);
+      const int d0 = wave * 64 + (MODE == kAffine && BITS == 8 ? j * 16 + s * 8 : s * 32 + j * 8);
+      bqh[rt][s] = *reinterpret_cast<const half8_t*>(qhi + row * QS + d0);
+      if constexpr (MODE != kPlain) bql[rt][s] = *reinterpret_cast<const half8_t*>(qlo + row * QS + d0);
     }
-    qs[gi] = MODE == kAffine ? qsum[row * NG + g] : 0.0f;
+    qs[rt] = MODE == kAffine ? qsum[row * NG + wave] : 0.0f;
   }
-  __syncthreads();  // the table is consumed: the region becomes the stages
-  // codebook: the centroid lookup table, after the stages (written before
-  // the first block's barrier)
+  __syncthreads();  // the table is consumed: the region becomes the buffers
   uint8_t* const lut = region + P::kLutOff;
   const uint32_t lut_l = lds_addr(lut) + (lane & (kLutCopies - 1)) * 4;
-  if constexpr (MODE == kCodebook) cb_fill_lut<CB>(lut, tid, kPfWaves * 64);
+  if constexpr (MODE == kCodebook) {
+    cb_fill_lut<CB>(lut, tid, NW * 64);
+    __syncthreads();
+  }
 
-  // ---- copies ----
-  const uint32_t stage_lds = lds_addr(region);
-  auto copy_vb = [&](int st, int i) {
-    const u32x4 rs = buffer_rsrc(blk_ptr(i), (uint32_t)P::kBytes);
-    const uint32_t sl = stage_lds + st * SB;
+  // ---- this wave's loads: the codes (and scale / bias) of its 64 dims in
+  // the two blocks of a step ----
+  uint32_t kr[2][KW], vr[2][VW];
+  u32x4 km[2], vm[2];
+  const int kbit = (c * (D / 2) + (wave % (NG / 2)) * 64 + 8 * j) * CB;
+  const int vbit = (c * 16 + 4 * j) * CB;
+  const uint32_t ksh = kbit & 31, vsh = vbit & 31;
+  const uint32_t k_off =
+      (int)L.k_codes +
+      (MODE == kAffine     ? (BITS == 8 ? wave * 1024 + lane * 16 : (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8)
+       : MODE == kCodebook ? (wave / (NG / 2)) * (D * CB) + (kbit >> 5) * 4
+                           : (c * D + wave * 64 + 8 * j) * 2);
+  const uint32_t v_off =
+      (int)L.v_codes +
+      (MODE == kAffine     ? (BITS == 8 ? wave * 1024 + lane * 16 : (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8)
+       : MODE == kCodebook ? wave * (128 * CB) + (vbit >> 5) * 4
+                           : ((wave * 64 + c) * kBlockTokens + 4 * j) * 2);
+  const uint32_t km_off = (int)L.k_meta + wave * 64 + j * 16;  // affine
+  const uint32_t vm_off = (int)L.v_meta + wave * 64 + j * 16;
+  auto load_k = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < CP; k++) {
-      const int ci = wave + kPfWaves * k;
-      dma16(sl + ci * kChunk, ci * kChunk + lane * 16, rs);
-    }
-  };
+    for (int kt = 0; kt < 2; kt++) {
+      if constexpr (MODE == kAffine) {
+        if constexpr (BITS == 8) {
+          const u32x4 w = load_at<u32x4>(bp[kt], k_off);
 #pragma unroll
-  for (int s = 0; s < NST - 1; s++)
-    if (s < nvb) copy_vb(s, s);
-
-  // ---- main loop ----
-  float4_t o[GH * 4];
-#pragma unroll
-  for (int i = 0; i < GH * 4; i++) o[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  float bacc[GH], psum[GH];
-#pragma unroll
-  for (int gi = 0; gi < GH; gi++) bacc[gi] = psum[gi] = 0.0f;
-  float m_run = -1e30f, l_run = 0.0f;
-  float neg_one;
-  asm("v_mov_b32 %0, -1.0" : "=v"(neg_one));
-
-  auto codes = [&](const uint8_t* sp, int region_off, int gi) {
-    const int g = g0 + gi;
-    return lds16(sp + region_off + (BITS == 8 ? g : g / 2) * kChunk + lane * 16);
-  };
-  auto kmeta = [&](const uint8_t* sp, int gi) {
-    return lds16(sp + (int)L.k_meta + (g0 + gi) * 64 + j * 16);
-  };
-  auto vmeta = [&](const uint8_t* sp, int gi) {
-    return lds16(sp + (int)L.v_meta + (g0 + gi) * 64 + j * 16);
-  };
-
-  // codebook: this lane's index fields in the wave's half of K (token c,
-  // dims 8 j .. of each slice) and V (dim c of each tile, tokens 4 j ..)
-  constexpr int HB = D * CB;  // bytes of one half of the K (or V) indices
-  const int kbit0 = (c * (D / 2) + 8 * j) * CB, vbit0 = (c * 16 + 4 * j) * CB;
-  const uint32_t ksh = kbit0 & 31, vsh = vbit0 & 31;
-  // plain: this lane's operand offsets (K row c, dims 8 j .. of each slice;
-  // V dim c of each tile, tokens 4 j ..)
-  const int pk_off = (int)L.k_codes + (c * D + half * (D / 2) + 8 * j) * 2;
-  const int pv_off = (int)L.v_codes + ((half * (D / 2) + c) * kBlockTokens + 4 * j) * 2;
-
-  auto process = [&](const uint8_t* sp, int vi, int it, bool full) {
-    float4_t sv = (float4_t){0.f, 0.f, 0.f, 0.f};
-    if constexpr (MODE == kCodebook) {
-      const uint32_t* kw =
-          reinterpret_cast<const uint32_t*>(sp + (int)L.k_codes + half * HB) + (kbit0 >> 5);
-#pragma unroll
-      for (int k = 0; k < NSW; k++) {
-        const uint32_t f = lds_field<CB>(kw, k * CB, ksh);
-        if constexpr (kCbExact<CB>) {
-          const half8_t ak = __builtin_bit_cast(
-              half8_t, (u32x4){cb_pair_exact<CB, 0>(lut_l, f), cb_pair_exact<CB, 1>(lut_l, f),
-                               cb_pair_exact<CB, 2>(lut_l, f), cb_pair_exact<CB, 3>(lut_l, f)});
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bqh[k >> 1][k & 1], sv, 0, 0, 0);
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(ak, bql[k >> 1][k & 1], sv, 0, 0, 0);
+          for (int i = 0; i < 4; i++) kr[kt][i] = w[i];
         } else {
-          uint32_t h4[4], l4[4];
-          cb_pair_hl4<0>(lut_l, f, h4[0], l4[0]);
-          cb_pair_hl4<1>(lut_l, f, h4[1], l4[1]);
-          cb_pair_hl4<2>(lut_l, f, h4[2], l4[2]);
-          cb_pair_hl4<3>(lut_l, f, h4[3], l4[3]);
-          const half8_t ah = __builtin_bit_cast(half8_t, (u32x4){h4[0], h4[1], h4[2], h4[3]});
-          const half8_t al = __builtin_bit_cast(half8_t, (u32x4){l4[0], l4[1], l4[2], l4[3]});
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bqh[k >> 1][k & 1], sv, 0, 0, 0);
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bqh[k >> 1][k & 1], sv, 0, 0, 0);
-          sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bql[k >> 1][k & 1], sv, 0, 0, 0);
+          const u32x2 w = load_at<u32x2>(bp[kt], k_off);
+          kr[kt][0] = w[0];
+          kr[kt][1] = w[1];
+        }
+        km[kt] = load_at<u32x4>(bp[kt], km_off);
+      } else if constexpr (MODE == kCodebook) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          if constexpr (CB == 3) {
+            const u32x2 w = load_at<u32x2_a4>(bp[kt], k_off + s * 4 * CB);
+            kr[kt][2 * s] = w[0];
+            kr[kt][2 * s + 1] = w[1];
+          } else {
+            kr[kt][s] = load_at<uint32_t>(bp[kt], k_off + s * 4 * CB);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const u32x4 w = load_at<u32x4>(bp[kt], k_off + s * 64);
+#pragma unroll
+          for (int i = 0; i < 4; i++) kr[kt][4 * s + i] = w[i];
         }
       }
-    } else if constexpr (MODE == kPlain) {
-#pragma unroll
-      for (int k = 0; k < NSW; k++)
-        sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8_t, lds16(sp + pk_off + k * 64)),
-            __builtin_bit_cast(bf16x8_t, bqh[k >> 1][k & 1]), sv, 0, 0, 0);
-    } else {
-    u32x4 kw = codes(sp, (int)L.k_codes, 0), km = kmeta(sp, 0);
-#pragma unroll
-    for (int gi = 0; gi < GH; gi++) {
-      const u32x4 kw_g = kw, km_g = km;
-      if (gi + 1 < GH) {
-        if (BITS == 8 || ((g0 + gi + 1) & 1) == 0) kw = codes(sp, (int)L.k_codes, gi + 1);
-        km = kmeta(sp, gi + 1);
-      }
-      const int g = g0 + gi;
-      const half8_t k0 = k_operand_plain<BITS>(kw_g, g, 0), k1 = k_operand_plain<BITS>(kw_g, g, 1);
-      const float4_t z = (float4_t){0.f, 0.f, 0.f, 0.f};
-      // the residual products first, then the high parts, in one accumulator
-      float4_t acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, bql[gi][0], z, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, bql[gi][1], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, bqh[gi][0], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, bqh[gi][1], acc, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        sv[i] = fmaf(lo16(km_g[i]), acc[i], fmaf(hi16(km_g[i]), qs[gi], sv[i]));
-      __builtin_amdgcn_sched_barrier(0);
     }
-    }
-
-    // exchange the half scores with the partner wave (release / acquire on
-    // a per-wave counter); both waves add the halves in the same order
-    const int par = it & 1;
-    xs[(wave * 2 + par) * 64 + lane] = sv;
-    __hip_atomic_store(&xflag[wave], it + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    while (__hip_atomic_load(&xflag[wave ^ 1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
-           it + 1)
-      __builtin_amdgcn_s_sleep(1);
-    const float4_t so = xs[((wave ^ 1) * 2 + par) * 64 + lane];
-    const float4_t s0 = half == 0 ? sv : so;
-    const float4_t s1 = half == 0 ? so : sv;
-    float s[4];
+  };
+  auto load_v = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) s[i] = s0[i] + s1[i];
-    // codebook: the keys' norms / sqrt(D) (lane (j, c) holds keys 4 j ..);
-    // plain: the softmax scale
-    float vscale[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (MODE == kCodebook) {
-      const uint2 kn = *reinterpret_cast<const uint2*>(sp + (int)L.k_meta + 8 * j);
-      const uint2 vn = *reinterpret_cast<const uint2*>(sp + (int)L.v_meta + 8 * j);
-      const float ks[4] = {lo16(kn.x), hi16(kn.x), lo16(kn.y), hi16(kn.y)};
-      const float vs[4] = {lo16(vn.x), hi16(vn.x), lo16(vn.y), hi16(vn.y)};
-      // (1 / sqrt(D) in the table operands' units)
-      const float cu = a.c * kCbOperandScale<CB>;
+    for (int kt = 0; kt < 2; kt++) {
+      if constexpr (MODE == kAffine) {
+        if constexpr (BITS == 8) {
+          const u32x4 w = load_at<u32x4>(bp[kt], v_off);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        s[i] = s[i] * (ks[i] * cu);
-        vscale[i] = vs[i] * cu;
-      }
-    } else if constexpr (MODE == kPlain) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) s[i] = s[i] * a.qscale;
-    }
-
-    // masks: the whole block for all rows of the pair in the common case
-    if (!full) {
-      const VB v = vb_of(vi);
-      const int64_t t0 = v.b * kBlockTokens;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int64_t kp = t0 + 4 * j + i;
-        const bool vis = row_valid && kp >= v.vlo && kp < v.vhi && kp >= row_lo && kp <= p_row;
-        if (!vis) s[i] = -INFINITY;
-      }
-    }
-    float mb = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    mb = xor16_max(mb);
-    mb = xor32_max(mb);
-    const float m_new = fmaxf(m_run, mb);
-    if (__any(m_new > m_run + kRescaleSlack)) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      if (__any(l_run > 0.0f)) {
-#pragma unroll
-        for (int i = 0; i < GH * 4; i++) o[i] *= alpha;
-#pragma unroll
-        for (int gi = 0; gi < GH; gi++) {
-          bacc[gi] *= alpha;
-          if constexpr (MODE == kAffine && kBiasedCodes<BITS>) psum[gi] *= alpha;
-        }
-      }
-      l_run *= alpha;
-      m_run = m_new;
-    }
-    float p[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) p[i] = __builtin_amdgcn_exp2f(s[i] - m_run);
-    l_run += (p[0] + p[1]) + (p[2] + p[3]);
-
-    if constexpr (MODE == kCodebook) {
-      // O^T += V^T . P'^T, P' = p * norm / sqrt D as f16 high part and
-      // residual, the centroids likewise
-      float x[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) x[i] = p[i] * vscale[i];
-      const half2_t h01 = pkrtz(x[0], x[1]);
-      const half2_t h23 = pkrtz(x[2], x[3]);
-      const half2_t r01 = pkrtz(fmaf(neg_one, (float)h01[0], x[0]), fmaf(neg_one, (float)h01[1], x[1]));
-      const half2_t r23 = pkrtz(fmaf(neg_one, (float)h23[0], x[2]), fmaf(neg_one, (float)h23[1], x[3]));
-      const half4_t bh = cat4(h01, h23), bl = cat4(r01, r23);
-      const uint32_t* vw =
-          reinterpret_cast<const uint32_t*>(sp + (int)L.v_codes + half * HB) + (vbit0 >> 5);
-#pragma unroll
-      for (int n = 0; n < NTW; n++) {
-        const uint32_t f = lds_field<CB>(vw, n * 8 * CB, vsh);
-        if constexpr (kCbExact<CB>) {
-          const half4_t av = __builtin_bit_cast(
-              half4_t, make_uint2(cb_pair_exact<CB, 0>(lut_l, f), cb_pair_exact<CB, 1>(lut_l, f)));
-          o[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bh, o[n], 0, 0, 0);
-          o[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bl, o[n], 0, 0, 0);
+          for (int i = 0; i < 4; i++) vr[kt][i] = w[i];
         } else {
-          uint32_t h2[2], l2[2];
-          cb_pair_hl4<0>(lut_l, f, h2[0], l2[0]);
-          cb_pair_hl4<1>(lut_l, f, h2[1], l2[1]);
-          const half4_t ah = __builtin_bit_cast(half4_t, make_uint2(h2[0], h2[1]));
-          const half4_t al = __builtin_bit_cast(half4_t, make_uint2(l2[0], l2[1]));
-          o[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bh, o[n], 0, 0, 0);
-          o[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(al, bh, o[n], 0, 0, 0);
-          o[n] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bl, o[n], 0, 0, 0);
+          const u32x2 w = load_at<u32x2>(bp[kt], v_off);
+          vr[kt][0] = w[0];
+          vr[kt][1] = w[1];
+        }
+        vm[kt] = load_at<u32x4>(bp[kt], vm_off);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+          if constexpr (MODE == kCodebook && CB != 3) {
+            vr[kt][n] = load_at<uint32_t>(bp[kt], v_off + n * 32 * CB);
+          } else {
+            const u32x2 w =
+                MODE == kCodebook ? (u32x2)load_at<u32x2_a4>(bp[kt], v_off + n * 32 * CB)
+                                  : load_at<u32x2>(bp[kt], v_off + n * 16 * kBlockTokens * 2);
+            vr[kt][2 * n] = w[0];
+            vr[kt][2 * n + 1] = w[1];
+          }
         }
       }
-      return;
-    } else if constexpr (MODE == kPlain) {
-      // O^T += V^T . P^T, P as bf16 high part and residual
-      float r[4];
+    }
+  };
+  // codebook: the key norms of a step's softmax stage (K and V), the lane's
+  // own quads
+  u32x2 kn[NQ], vn[NQ];
+  const int quad0 = kOwn ? j : lane >> 3;  // the lane's first key quad (then quad0 + 4)
+  auto load_n = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
+    if constexpr (MODE == kCodebook) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) r[i] = p[i] - bf16_to_f32(f32_to_bf16(p[i]));
-      const short4_t bh = __builtin_bit_cast(
-          short4_t, make_uint2(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3])));
-      const short4_t bl = __builtin_bit_cast(
-          short4_t, make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])));
-#pragma unroll
-      for (int n = 0; n < NTW; n++) {
-        const short4_t va =
-            __builtin_bit_cast(short4_t, *reinterpret_cast<const uint2*>(sp + pv_off + n * 16 * kBlockTokens * 2));
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, bh, o[n], 0, 0, 0);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, bl, o[n], 0, 0, 0);
+      for (int u = 0; u < NQ; u++) {
+        const gptr_t p = (kOwn ? u == 0 : quad0 < 4) ? bp[0] : bp[1];
+        kn[u] = load_at<u32x2>(p, (uint32_t)L.k_meta + 8 * (quad0 & 3));
+        vn[u] = load_at<u32x2>(p, (uint32_t)L.v_meta + 8 * (quad0 & 3));
       }
-      return;
-    } else {
-    u32x4 vw = codes(sp, (int)L.v_codes, 0), vm = vmeta(sp, 0);
+    }
+  };
 
-    // O^T += V^T . P'^T, P' = p * v_scale as f16 high part and residual
-    const half2_t one2 = (half2_t){(_Float16)1.0f, (_Float16)1.0f};
+  // ---- the three stages ----
+  float4_t o[kPfTiles][4];  // [row tile][dim tile]: dims 16 ct + 4 j .., row 16 rt + c
+  float bacc[kPfTiles];
 #pragma unroll
-    for (int gi = 0; gi < GH; gi++) {
-      const u32x4 vw_g = vw, vm_g = vm;
-      if (gi + 1 < GH) {
-        if (BITS == 8 || ((g0 + gi + 1) & 1) == 0) vw = codes(sp, (int)L.v_codes, gi + 1);
-        vm = vmeta(sp, gi + 1);
-      }
-      float x[4];
+  for (int rt = 0; rt < kPfTiles; rt++) {
+    bacc[rt] = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        x[i] = fmaf(p[i], lo16(vm_g[i]), 0.0f);
-        bacc[gi] = fmaf(p[i], hi16(vm_g[i]), bacc[gi]);
+    for (int ct = 0; ct < 4; ct++) o[rt][ct] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  }
+  float m_run[NRS], l_run[NRS];
+#pragma unroll
+  for (int u = 0; u < NRS; u++) m_run[u] = -1e30f, l_run[u] = 0.0f;
+  float4_t own[NRS][2];  // this wave's partial of the rows it sums (kOwn)
+  // row of softmax row set u
+  auto sm_row = [&](int u) __attribute__((always_inline)) { return kOwn ? (wave * NRS + u) * 16 + c : wave * 8 + (lane & 7); };
+
+  int p_row[NRS];  // the row's position
+#pragma unroll
+  for (int u = 0; u < NRS; u++) p_row[u] = pA_r + sm_row(u) / G;
+
+  float4_t* const xs = reinterpret_cast<float4_t*>(region);
+  u32x4* const pb = reinterpret_cast<u32x4*>(region + P::kPbOff);
+  float* const al = reinterpret_cast<float*>(region + P::kAlOff);
+
+  auto qk = [&](int buf) __attribute__((always_inline)) {
+    float4_t* const xb = xs + buf * (P::kXs / 16) + lane;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      float4_t acc[kPfTiles];
+#pragma unroll
+      for (int rt = 0; rt < kPfTiles; rt++) acc[rt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+      if constexpr (MODE == kPlain) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const bf16x8_t ak = __builtin_bit_cast(
+              bf16x8_t, (u32x4){kr[kt][4 * s], kr[kt][4 * s + 1], kr[kt][4 * s + 2], kr[kt][4 * s + 3]});
+#pragma unroll
+          for (int rt = 0; rt < kPfTiles; rt++)
+            acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                ak, __builtin_bit_cast(bf16x8_t, bqh[rt][s]), acc[rt], 0, 0, 0);
+        }
+      } else {
+        half8_t ah[2], alo[2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          if constexpr (MODE == kAffine) {
+            ah[s] = k_operand_plain<BITS>(kr[kt], s);
+          } else {
+            uint32_t f;
+            if constexpr (CB == 3)
+              f = __builtin_amdgcn_alignbit(kr[kt][2 * s + 1], kr[kt][2 * s], ksh);
+            else
+              f = kr[kt][s] >> ksh;
+            if constexpr (kCbExact<CB>) {
+              ah[s] = __builtin_bit_cast(
+                  half8_t, (u32x4){cb_pair_exact<CB, 0>(lut_l, f), cb_pair_exact<CB, 1>(lut_l, f),
+                                   cb_pair_exact<CB, 2>(lut_l, f), cb_pair_exact<CB, 3>(lut_l, f)});
+            } else {
+              uint32_t h4[4], l4[4];
+              cb_pair_hl4<0>(lut_l, f, h4[0], l4[0]);
+              cb_pair_hl4<1>(lut_l, f, h4[1], l4[1]);
+              cb_pair_hl4<2>(lut_l, f, h4[2], l4[2]);
+              cb_pair_hl4<3>(lut_l, f, h4[3], l4[3]);
+              ah[s] = __builtin_bit_cast(half8_t, (u32x4){h4[0], h4[1], h4[2], h4[3]});
+              alo[s] = __builtin_bit_cast(half8_t, (u32x4){l4[0], l4[1], l4[2], l4[3]});
+            }
+          }
+        }
+        // the residual products first, then the high parts, in one accumulator
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+          for (int rt = 0; rt < kPfTiles; rt++)
+            acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bql[rt][s], acc[rt], 0, 0, 0);
+        if constexpr (MODE == kCodebook && !kCbExact<CB>) {
+#pragma unroll
+          for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int rt = 0; rt < kPfTiles; rt++)
+              acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[s], bqh[rt][s], acc[rt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+          for (int rt = 0; rt < kPfTiles; rt++)
+            acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bqh[rt][s], acc[rt], 0, 0, 0);
       }
-      const half2_t h01 = pkrtz(x[0], x[1]);
-      const half2_t h23 = pkrtz(x[2], x[3]);
-      // residual x - hi (exact) as one mixed-precision fma each (an opaque
-      // -1 keeps the f16 operand inside the fma instead of a convert and a
-      // subtract)
-      const half2_t r01 = pkrtz(fmaf(neg_one, (float)h01[0], x[0]), fmaf(neg_one, (float)h01[1], x[1]));
-      const half2_t r23 = pkrtz(fmaf(neg_one, (float)h23[0], x[2]), fmaf(neg_one, (float)h23[1], x[3]));
-      const half4_t bh = cat4(h01, h23), bl = cat4(r01, r23);
-      if constexpr (kBiasedCodes<BITS>) {
-        float t = __builtin_amdgcn_fdot2(h01, one2, psum[gi], false);
-        t = __builtin_amdgcn_fdot2(h23, one2, t, false);
-        t = __builtin_amdgcn_fdot2(r01, one2, t, false);
-        psum[gi] = __builtin_amdgcn_fdot2(r23, one2, t, false);
+#pragma unroll
+      for (int rt = 0; rt < kPfTiles; rt++) {
+        float4_t sv = acc[rt];
+        if constexpr (MODE == kAffine) {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            sv[i] = fmaf(lo16(km[kt][i]), acc[rt][i], hi16(km[kt][i]) * qs[rt]);
+        }
+        if constexpr (kOwn) {
+          const int owner = rt / NRS;  // the wave that sums this row tile
+          if (owner == wave)
+            own[rt % NRS][kt] = sv;
+          else
+            xb[((rt * P::kSrc + (wave < owner ? wave : wave - 1)) * 2 + kt) * 64] = sv;
+        } else {
+          xb[((wave * 2 + kt) * kPfTiles + rt) * 64] = sv;
+        }
       }
-      const int g = g0 + gi;
+    }
+  };
+
+  auto softmax = [&](int buf, int step, const float4_t (&mine)[NRS][2], bool full) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NRS; u++) {
+      const int row = sm_row(u);
+      float s[NQ][4];
+      if constexpr (kOwn) {
+        const float4_t* xr = xs + buf * (P::kXs / 16) + (wave * NRS + u) * P::kSrc * 128 + lane;
+#pragma unroll
+        for (int t = 0; t < NQ; t++) {
+          float4_t v = mine[u][t];
+#pragma unroll
+          for (int g = 0; g < P::kSrc; g++) v += xr[(g * 2 + t) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; i++) s[t][i] = v[i];
+        }
+      } else {
+        const float4_t* xr = xs + buf * (P::kXs / 16) +
+                             ((quad0 >> 2) * kPfTiles + (wave >> 1)) * 64 + (quad0 & 3) * 16 +
+                             (wave & 1) * 8 + (lane & 7);
+        float4_t v = xr[0];
+#pragma unroll
+        for (int g = 1; g < NG; g++) v += xr[g * 2 * kPfTiles * 64];
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[0][i] = v[i];
+      }
+      // codebook: the keys' norms / sqrt(D); plain: the softmax scale
+      float vscale[NQ][4];
+      if constexpr (MODE == kCodebook) {
+        // (1 / sqrt(D) in the table operands' units)
+        const float cu = a.c * kCbOperandScale<CB>;
+#pragma unroll
+        for (int t = 0; t < NQ; t++) {
+          const float ks[4] = {lo16(kn[t][0]), hi16(kn[t][0]), lo16(kn[t][1]), hi16(kn[t][1])};
+          const float vs[4] = {lo16(vn[t][0]), hi16(vn[t][0]), lo16(vn[t][1]), hi16(vn[t][1])};
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            s[t][i] = s[t][i] * (ks[i] * cu);
+            vscale[t][i] = vs[i] * cu;
+          }
+        }
+      } else if constexpr (MODE == kPlain) {
+#pragma unroll
+        for (int t = 0; t < NQ; t++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) s[t][i] = s[t][i] * a.qscale;
+      }
+      if (!full) {
+        const int p = p_row[u], lo = lo_rel(p);
+#pragma unroll
+        for (int t = 0; t < NQ; t++) {
+          const int vi = 2 * step + (kOwn ? t : quad0 >> 2);
+          int vlo, vhi;
+          vb_range(vi, vlo, vhi);
+          vlo = vlo > lo ? vlo : lo;
+          vhi = vhi < p + 1 ? vhi : p + 1;
+          const int kp = (vi < n_old_i ? vi : vi + vb_shift) * kBlockTokens + 4 * (quad0 & 3);
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (!(kp + i >= vlo && kp + i < vhi)) s[t][i] = -INFINITY;
+        }
+      }
+      float mb = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NQ; t++)
+        mb = fmaxf(mb, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
+      if constexpr (!kOwn) mb = fmaxf(mb, row_ror8(mb));
+      mb = xor16_max(mb);
+      mb = xor32_max(mb);
+      const float m_new = fmaxf(m_run[u], mb);
+      const float m_old = m_run[u];
+      m_run[u] = __any(m_new > m_old + kRescaleSlack) ? m_new : m_old;
+      const float alpha = __builtin_amdgcn_exp2f(m_old - m_run[u]);  // 1 when it stays
+      l_run[u] *= alpha;
+      if (kOwn ? j == 0 : lane < 8) al[buf * kPfRows + (row & 15) * 4 + (row >> 4)] = alpha;
+#pragma unroll
+      for (int t = 0; t < NQ; t++) {
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[i] = __builtin_amdgcn_exp2f(s[t][i] - m_run[u]);
+        l_run[u] += (p[0] + p[1]) + (p[2] + p[3]);
+        asm volatile("" : "+v"(l_run[u]));
+        u32x4 w;
+        if constexpr (MODE != kPlain) {
+          // f16 high part and residual of P (affine) or of P' = p * norm /
+          // sqrt D (codebook)
+          half4_t h, r;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            float x = MODE == kCodebook ? p[i] * vscale[t][i] : p[i];
+            // (one rounded product for both parts: fused into either conversion
+            // it can round the high part to its other neighbour)
+            asm("" : "+v"(x));
+            h[i] = (_Float16)x;
+            r[i] = (_Float16)(x - (float)h[i]);
+          }
+          const uint2 hw = __builtin_bit_cast(uint2, h), rw = __builtin_bit_cast(uint2, r);
+          w = (u32x4){hw.x, hw.y, rw.x, rw.y};
+        } else {
+          // P as bf16 high part and residual
+          float r[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) r[i] = p[i] - bf16_to_f32(f32_to_bf16(p[i]));
+          w = (u32x4){pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(r[0], r[1]),
+                      pack_bf16x2(r[2], r[3])};
+        }
+        pb[buf * (P::kPb / 16) + (quad0 + 4 * t) * kPfRows + row] = w;
+      }
+    }
+  };
+
+  auto rescale = [&](int buf) __attribute__((always_inline)) {
+    const float4_t av = *reinterpret_cast<const float4_t*>(al + buf * kPfRows + c * 4);
+    if (__any(av[0] != 1.0f || av[1] != 1.0f || av[2] != 1.0f || av[3] != 1.0f)) {
+#pragma unroll
+      for (int rt = 0; rt < kPfTiles; rt++) {
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) o[rt][ct] *= av[rt];
+        bacc[rt] *= av[rt];
+      }
+    }
+  };
+  auto pv = [&](int buf) __attribute__((always_inline)) {
+    half2_t vsc[4], vbi[4];  // affine: scales and biases of the lane's key pairs
+    if constexpr (MODE == kAffine) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t m0 = vm[e >> 1][(e & 1) * 2], m1 = vm[e >> 1][(e & 1) * 2 + 1];
+        vsc[e] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(m1, m0, 0x05040100u));
+        vbi[e] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(m1, m0, 0x07060302u));
+      }
+    }
+    // V operands of the four dim tiles (codebook 4 bits: high parts and residuals)
+    half8_t va[4], vl[4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) {
+      if constexpr (MODE == kAffine) {
+        va[ct] = v_operand_plain<BITS>(vr[0], vr[1], ct);
+      } else if constexpr (MODE == kPlain) {
+        va[ct] = __builtin_bit_cast(
+            half8_t, (u32x4){vr[0][2 * ct], vr[0][2 * ct + 1], vr[1][2 * ct], vr[1][2 * ct + 1]});
+      } else {
+        uint32_t f[2], h[4], l[4];
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+          if constexpr (CB == 3)
+            f[kt] = __builtin_amdgcn_alignbit(vr[kt][2 * ct + 1], vr[kt][2 * ct], vsh);
+          else
+            f[kt] = vr[kt][ct] >> vsh;
+          if constexpr (kCbExact<CB>) {
+            h[2 * kt] = cb_pair_exact<CB, 0>(lut_l, f[kt]);
+            h[2 * kt + 1] = cb_pair_exact<CB, 1>(lut_l, f[kt]);
+          } else {
+            cb_pair_hl4<0>(lut_l, f[kt], h[2 * kt], l[2 * kt]);
+            cb_pair_hl4<1>(lut_l, f[kt], h[2 * kt + 1], l[2 * kt + 1]);
+          }
+        }
+        va[ct] = __builtin_bit_cast(half8_t, (u32x4){h[0], h[1], h[2], h[3]});
+        if constexpr (!kCbExact<CB>)
+          vl[ct] = __builtin_bit_cast(half8_t, (u32x4){l[0], l[1], l[2], l[3]});
+      }
+    }
+#pragma unroll
+    for (int rt = 0; rt < kPfTiles; rt++) {
+      const u32x4 w0 = pb[buf * (P::kPb / 16) + j * kPfRows + rt * 16 + c];
+      const u32x4 w1 = pb[buf * (P::kPb / 16) + (j + 4) * kPfRows + rt * 16 + c];
+      half8_t bh, bl;
+      if constexpr (MODE == kAffine) {
+        // P' = p * v_scale in packed f16: the high part P_hi * s rounded, then
+        // its exact rounding error plus P_lo * s
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const half2_t ph = __builtin_bit_cast(half2_t, e < 2 ? w0[e] : w1[e - 2]);
+          const half2_t pl = __builtin_bit_cast(half2_t, e < 2 ? w0[e + 2] : w1[e]);
+          const half2_t h = ph * vsc[e];
+          const half2_t l = __builtin_elementwise_fma(
+              pl, vsc[e], __builtin_elementwise_fma(ph, vsc[e], -h));
+          bh[2 * e] = h[0];
+          bh[2 * e + 1] = h[1];
+          bl[2 * e] = l[0];
+          bl[2 * e + 1] = l[1];
+          bacc[rt] = __builtin_amdgcn_fdot2(pl, vbi[e], bacc[rt], false);
+          bacc[rt] = __builtin_amdgcn_fdot2(ph, vbi[e], bacc[rt], false);
+        }
+        // (here, not sunk past the barrier with every weight and bias kept for it)
+        asm volatile("" : "+v"(bacc[rt]));
+      } else {
+        bh = __builtin_bit_cast(half8_t, (u32x4){w0[0], w0[1], w1[0], w1[1]});
+        bl = __builtin_bit_cast(half8_t, (u32x4){w0[2], w0[3], w1[2], w1[3]});
+      }
 #pragma unroll
       for (int ct = 0; ct < 4; ct++) {
-        const half4_t va = v_operand<BITS>(vw_g, g, ct);
-        o[gi * 4 + ct] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, bh, o[gi * 4 + ct], 0, 0, 0);
-        o[gi * 4 + ct] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, bl, o[gi * 4 + ct], 0, 0, 0);
+        if constexpr (MODE == kPlain) {
+          const bf16x8_t v = __builtin_bit_cast(bf16x8_t, va[ct]);
+          o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8_t, bh),
+                                                              o[rt][ct], 0, 0, 0);
+          o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8_t, bl),
+                                                              o[rt][ct], 0, 0, 0);
+        } else {
+          o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[ct], bh, o[rt][ct], 0, 0, 0);
+          if constexpr (MODE == kCodebook && !kCbExact<CB>)
+            o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[ct], bh, o[rt][ct], 0, 0, 0);
+          o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[ct], bl, o[rt][ct], 0, 0, 0);
+        }
       }
-    }
     }
   };
 
-  int st = 0, it = 0;
-  for (int i = 0; i < nvb; i++) {
-    // this wave's copies of block i have landed (only the blocks issued
-    // after it may be pending); the barrier makes every wave's copies
-    // visible and frees the stage of block i - 1 for block i + NST - 1
-    const int rest = nvb - 1 - i;
-    wait_copies<CP, NST - 2>(rest < NST - 2 ? rest : NST - 2);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (i + NST - 1 < nvb) copy_vb((i + NST - 1) % NST, i + NST - 1);
-    // the pair's rows see this block at all (pair-uniform)
-    const int rb = i < n_old ? i : new_rb0 + (i - (int)n_old);
-    bool sees = rb >= sees_lo && rb <= sees_hi;
-    if (rb == cut_rb) {
-      const VB v = vb_of(i);
-      sees = pair_any && v.vhi - 1 >= pair_lo_min && v.vlo <= pB;
+  // ---- the pipeline over steps s_begin .. s_end - 1 ----
+  const int s_begin = 0, s_end = nst;
+  const int n = s_end - s_begin;
+  gptr_t cur[2], nxt[2], after[2];  // the blocks of steps i, i + 1, i + 2
+  bool f_cur = false, f_nxt = false, f_after = false;
+  // the blocks of step s_begin + i (past the end: of the last one)
+  auto blocks_of = [&](int i, gptr_t (&bp)[2], bool& f) __attribute__((always_inline)) {
+    if (i >= n) i = n - 1;
+    const int v = 2 * (s_begin + i);
+    bp[0] = blk_ptr(v);
+    bp[1] = blk_ptr(v + 1);
+    f = blk_full(v) && blk_full(v + 1);
+  };
+  float4_t mine[NRS][2];
+  auto keep_own = [&]() __attribute__((always_inline)) {
+    if constexpr (kOwn) {
+#pragma unroll
+      for (int u = 0; u < NRS; u++) mine[u][0] = own[u][0], mine[u][1] = own[u][1];
     }
-    if (sees) {
-      const bool full = rb >= full_lo && rb <= full_hi && rb != cut_rb;
-      process(region + st * SB, i, it, full);
-      it++;
+  };
+  auto advance = [&](int i) __attribute__((always_inline)) {  // cur = step i, nxt, after
+#pragma unroll
+    for (int t = 0; t < 2; t++) cur[t] = nxt[t], nxt[t] = after[t];
+    f_cur = f_nxt, f_nxt = f_after;
+    blocks_of(i + 2, after, f_after);
+  };
+  if (n > 0) {
+    blocks_of(0, cur, f_cur);
+    blocks_of(1, nxt, f_nxt);
+    blocks_of(2, after, f_after);
+    load_k(cur);
+    load_n(cur);
+    // the first interval's PV is of zero weights and codes
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+#pragma unroll
+      for (int w = 0; w < VW; w++) vr[kt][w] = 0;
+      vm[kt] = (u32x4){0, 0, 0, 0};
     }
-    st = st + 1 == NST ? 0 : st + 1;
+    for (int i = tid; i < P::kPb / 16; i += NW * 64) pb[P::kPb / 16 + i] = (u32x4){0, 0, 0, 0};
+    if (tid < kPfRows) al[kPfRows + tid] = 1.0f;
+    qk(0);
+    keep_own();
+    load_k(nxt);
+    lds_barrier();
+    // an interval between two barriers: QK of step i + 1 (past the end: of the
+    // last blocks, for nothing), softmax of step i, PV of step i - 1
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+      rescale((i - 1) & 1);
+      qk((i + 1) & 1);
+      load_k(after);
+      softmax(i & 1, s_begin + i, mine, f_cur);
+      keep_own();
+      load_n(nxt);
+      pv((i - 1) & 1);
+      load_v(cur);
+      lds_barrier();
+      advance(i + 1);
+    }
+    rescale((n - 1) & 1);
+    pv((n - 1) & 1);
   }
 
   // ---- epilogue: normalise, inverse rotation, store ----
-  l_run = xor16_sum(l_run);
-  l_run = xor32_sum(l_run);
 #pragma unroll
-  for (int gi = 0; gi < GH; gi++) {
-    bacc[gi] = xor16_sum(bacc[gi]);
-    bacc[gi] = xor32_sum(bacc[gi]);
-    if constexpr (MODE == kAffine && kBiasedCodes<BITS>) {
-      // the V codes entered the MFMAs as 1024 + code
-      const float t = xor32_sum(xor16_sum(psum[gi]));
-      bacc[gi] = fmaf(-1024.0f, t, bacc[gi]);
-    }
+  for (int u = 0; u < NRS; u++) {
+    if constexpr (!kOwn) l_run[u] += row_ror8(l_run[u]);
+    l_run[u] = xor16_sum(l_run[u]);
+    l_run[u] = xor32_sum(l_run[u]);
+    if (kOwn ? j == 0 : lane < 8) lrow[sm_row(u)] = l_run[u];
   }
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the stages are free
+  lds_barrier();  // the buffers are free
   float* const Rr = reinterpret_cast<float*>(region);
-  // (tile n of the wave's half: dims half * D / 2 + 16 n + 4 j .., the
-  // affine group / column-tile order being the same dims)
 #pragma unroll
-  for (int gi = 0; gi < GH; gi++)
+  for (int rt = 0; rt < kPfTiles; rt++) {
+    if constexpr (MODE == kAffine) bacc[rt] = xor32_sum(xor16_sum(bacc[rt]));
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++) {
-      const int d = (g0 + gi) * 64 + ct * 16 + 4 * j;
-      *reinterpret_cast<float4_t*>(&Rr[row * RS + d]) =
-          MODE == kAffine ? o[gi * 4 + ct] + bacc[gi] : o[gi * 4 + ct];
-    }
-  if (half == 0 && j == 0) lrow[row] = l_run;
+    for (int ct = 0; ct < 4; ct++)
+      *reinterpret_cast<float4_t*>(&Rr[(rt * 16 + c) * RS + wave * 64 + ct * 16 + 4 * j]) =
+          MODE == kAffine ? o[rt][ct] + bacc[rt] : o[rt][ct];
+  }
   __syncthreads();
-#pragma unroll 1
-  for (int k = 0; k < kPfRows / kPfWaves; k++) {
-    const int r = wave + kPfWaves * k;
+#pragma unroll 2
+  for (int k = 0; k < kPfRows / NW; k++) {
+    const int r = wave + NW * k;
     const int rq_ = r / G, rh_ = r - (r / G) * G;
     if (rq_ >= nq) continue;
     const float l = lrow[r];
     float x[E];
-#pragma unroll
-    for (int i = 0; i < E; i++) x[i] = apply_sign(Rr[r * RS + lane * E + i], sbits, i);
     float cs = cs_lane;
     if constexpr (MODE != kPlain) {
+#pragma unroll
+      for (int i = 0; i < E; i++) x[i] = apply_sign(Rr[r * RS + lane * E + i], sbits, i);
       wave_fwht_signed<E>(x, lane);
     } else {  // no rotation: the row as accumulated
 #pragma unroll
@@ -683,7 +886,8 @@ template <int D, int BITS, int MODE>
 hipError_t launch_t(const PrefillArgs& a, hipStream_t s) {
   const int qp = kPfRows / a.group;
   dim3 grid((a.n_q + qp - 1) / qp, a.new_st.n_kv_heads, a.n_seqs);
-  hipLaunchKernelGGL((prefill_attn_kernel<D, BITS, MODE>), grid, dim3(kPfWaves * 64), 0, s, a);
+  hipLaunchKernelGGL((prefill_attn_kernel<D, BITS, MODE>), grid,
+                     dim3(PfPlan<D, BITS, MODE>::NW * 64), 0, s, a);
   return hipGetLastError();
 }
 
