@@ -191,6 +191,19 @@ struct Workspace {
   }
 };
 
+// The partials of a handle's split prefill calls. Calls on several streams
+// may be in flight (a prefill never needed a workspace of the handle before
+// its grid was split), so each use waits, on its stream, for the one before.
+struct PrefillScratch {
+  Workspace ws;
+  hipEvent_t used = nullptr;
+  void release() {
+    ws.release();
+    if (used) (void)hipEventDestroy(used);
+    used = nullptr;
+  }
+};
+
 }  // namespace
 
 struct fmkv_cache {
@@ -205,6 +218,7 @@ struct fmkv_cache {
   int64_t vis_begin;
   Workspace ws;
   Workspace stage;  // prefill on a ring: the chunk's quantized rows
+  PrefillScratch split;
   int cus;
 };
 
@@ -217,6 +231,7 @@ struct fmkv_pool {
   uint32_t sign_bits[16];
   float c, sqrt_d;
   Workspace ws;
+  PrefillScratch split;
   int cus;
 };
 
@@ -246,6 +261,51 @@ fmkv::Store pool_store(const fmkv_pool* p, const int32_t* table, int32_t stride)
   s.n_kv_heads = p->desc.n_kv_heads;
   s.layout = p->layout;
   return s;
+}
+
+// The prefill attention, split over its keys when the grid alone would leave
+// CUs idle. Not under stream capture (the scratch may have to grow, and a
+// replay is not ordered with other uses of it) and not when there is no
+// memory for the partials: the unsplit launch needs none.
+hipError_t run_prefill(fmkv::PrefillArgs& pa, PrefillScratch& sc, int cus, int64_t max_steps,
+                       hipStream_t s) {
+  if (fmkv::prefill_is_short(pa, max_steps)) return fmkv::launch_prefill_short(pa, s);
+  size_t bytes = 0;
+  int units = fmkv::prefill_units(pa, cus, max_steps, &bytes);
+  if (units > 0) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      units = 0;
+    }
+  }
+  if (units > 0 && bytes > sc.ws.bytes) {
+    float* ptr = nullptr;
+    if (hipMalloc(&ptr, bytes) == hipSuccess) {
+      sc.ws.release();  // (hipFree waits for the calls that use it)
+      sc.ws.ptr = ptr;
+      sc.ws.bytes = bytes;
+    } else {
+      (void)hipGetLastError();
+      units = 0;
+    }
+  }
+  if (units > 0 && !sc.used && hipEventCreateWithFlags(&sc.used, hipEventDisableTiming) != hipSuccess) {
+    (void)hipGetLastError();
+    sc.used = nullptr;
+    units = 0;
+  }
+  if (units == 0) return fmkv::launch_prefill_attention(pa, s);
+  pa.units = units;
+  pa.part_o = sc.ws.ptr;
+  // (bytes = rows * (D + 2) floats)
+  const int D = pa.new_st.layout.head_dim;
+  pa.part_ml = sc.ws.ptr + bytes / sizeof(float) / (D + 2) * D;
+  hipError_t e = hipStreamWaitEvent(s, sc.used, 0);
+  if (e != hipSuccess) return e;
+  e = fmkv::launch_prefill_attention(pa, s);
+  if (e != hipSuccess) return e;
+  return hipEventRecord(sc.used, s);
 }
 
 int64_t visible_begin(const fmkv_cache* c) {
@@ -713,6 +773,7 @@ int fmkv_cache_destroy(fmkv_cache* c) {
   if (c->d_signs) (void)hipFree(c->d_signs);
   c->ws.release();
   c->stage.release();
+  c->split.release();
   delete c;
   return FMKV_OK;
 }
@@ -819,17 +880,20 @@ int fmkv_prefill_step(fmkv_cache* c, const void* k, const void* v, int64_t n, co
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
+  int64_t keys = p0 + n - c->vis_begin;
+  if (W > 0 && keys > W + 64) keys = W + 64;
+  const int64_t max_steps = keys / 32 + 2;
   if (W > 0) {
     e = fmkv::launch_append(as, 1, (int)nsb, s);
     if (e != hipSuccess) return hip_fail(e, "staging append launch");
-    e = fmkv::launch_prefill_attention(pa, s);
+    e = run_prefill(pa, c->split, c->cus, max_steps, s);
     if (e != hipSuccess) return hip_fail(e, "prefill attention launch");
     e = fmkv::launch_append(ap, 1, (int)tasks, s);
     if (e != hipSuccess) return hip_fail(e, "append launch");
   } else {
     e = fmkv::launch_append(ap, 1, (int)tasks, s);
     if (e != hipSuccess) return hip_fail(e, "append launch");
-    e = fmkv::launch_prefill_attention(pa, s);
+    e = run_prefill(pa, c->split, c->cus, max_steps, s);
     if (e != hipSuccess) return hip_fail(e, "prefill attention launch");
   }
   c->offset += n;
@@ -1033,6 +1097,7 @@ int fmkv_pool_destroy(fmkv_pool* p) {
   if (p->arena) (void)hipFree(p->arena);
   if (p->d_signs) (void)hipFree(p->d_signs);
   p->ws.release();
+  p->split.release();
   delete p;
   return FMKV_OK;
 }
@@ -1079,7 +1144,8 @@ int fmkv_paged_prefill_step(fmkv_pool* p, const void* k, const void* v,
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e = fmkv::launch_append(ap, n_seqs, tasks, s);
   if (e != hipSuccess) return hip_fail(e, "paged append launch");
-  e = fmkv::launch_prefill_attention(pa, s);
+  // (starts are on the device: the table's width bounds the lengths)
+  e = run_prefill(pa, p->split, p->cus, (int64_t)max_blocks / 2 + 2, s);
   if (e != hipSuccess) return hip_fail(e, "prefill attention launch");
   return FMKV_OK;
 }

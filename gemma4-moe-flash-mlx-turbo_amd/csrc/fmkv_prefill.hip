@@ -69,6 +69,14 @@
 // A paged pool runs one sequence per grid z with its own start position and
 // block table (linear sequences: the append goes first).
 //
+// A grid that would leave CUs idle is split over the keys as well (units > 0):
+// grid z then counts (sequence, key range) units instead of sequences, each
+// sequence getting a number of ranges that follows its length
+// (prefill_unit), and a second kernel merges the ranges' partial rows. Four
+// 77-token chunks after 700 .. 8000 positions (16 q / 2 KV heads of 512 dims,
+// 3-bit codebook: 80 work-groups, the longest of 253 steps): 0.196 ms against
+// 0.575 unsplit.
+//
 // Keys come from two stores: positions below p_split from old_st (the ring
 // of a sliding layer, read before the chunk's own append can overwrite
 // positions early queries still need), the rest from new_st (a staging
@@ -86,6 +94,15 @@ constexpr int kPfRows = 64;   // query rows per work-group, four matrix-core til
 constexpr int kPfTiles = kPfRows / 16;
 constexpr int kPfKeys = 2 * kBlockTokens;  // keys per step
 constexpr int kPfQuads = kPfKeys / 4;      // groups of four keys of a step
+constexpr int kPfMinSteps = 4;             // steps of the shortest key range of a split call
+
+// 2- and 3-bit codebook caches weigh V by p * norm / (1000 sqrt(D)), mostly
+// below 2^-8, where an f16 residual is subnormal and ends at 2^-25: their
+// weights carry a factor 32 that the accumulated row loses again (norm is an
+// f16, so p <= 2^8 and D >= 128 keep them below 4.8e4). Error against 64 bits
+// over 6000 positions: 1.8e-4 without it.
+template <int BITS>
+constexpr float kPvScale = kCbExact<BITS> ? 32.0f : 1.0f;
 
 template <int D, int BITS, int MODE>
 struct PfPlan {
@@ -162,10 +179,92 @@ __device__ inline T load_at(gptr_t p, uint32_t off) {
   return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off);
 }
 
+template <int N>
+__device__ inline void load_words(const uint16_t* src, uint32_t (&w)[N]) {
+  typedef uint32_t vec __attribute__((ext_vector_type(N == 1 ? 2 : N)));
+  if constexpr (N == 1) {
+    w[0] = *reinterpret_cast<const uint32_t*>(src);
+  } else {
+    const vec v = *reinterpret_cast<const vec*>(src);
+#pragma unroll
+    for (int i = 0; i < N; i++) w[i] = v[i];
+  }
+}
+
+// E consecutive outputs at element o_idx, in one store a lane (the caller's
+// buffer is aligned to its elements only).
+template <int E>
+__device__ inline void store_out(const PrefillArgs& a, int64_t o_idx, const float (&v)[E]) {
+  if (a.out_f32) {
+    typedef float vec __attribute__((ext_vector_type(E), aligned(4)));
+    vec o;
+#pragma unroll
+    for (int i = 0; i < E; i++) o[i] = v[i];
+    *reinterpret_cast<vec*>(reinterpret_cast<float*>(a.out) + o_idx) = o;
+  } else {
+    typedef uint16_t vec __attribute__((ext_vector_type(E), aligned(2)));
+    vec o;
+#pragma unroll
+    for (int i = 0; i < E; i++) o[i] = f32_to_bf16(v[i]);
+    *reinterpret_cast<vec*>(reinterpret_cast<uint16_t*>(a.out) + o_idx) = o;
+  }
+}
+
 // LDS of this wave written, every wave of the work-group here. Loads from
 // memory stay in flight across it.
 __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Steps (32 keys) that a row tile of a sequence may need, from its start.
+__device__ inline int prefill_steps(const PrefillArgs& a, int64_t p0) {
+  const int64_t lo = a.vis_begin > 0 ? a.vis_begin : 0;
+  int64_t keys = p0 + a.n_q - lo;
+  if (a.window > 0 && keys > a.window + kPfRows) keys = a.window + kPfRows;
+  if (keys > ((int64_t)1 << 25)) keys = (int64_t)1 << 25;  // (64 sequences' steps add up in 32 bits)
+  return (int)((keys > 0 ? keys : 0) / kPfKeys) + 2;
+}
+
+// What unit u of the grid is: its sequence, the sequence's first unit and its
+// number of key ranges. The range length c is the smallest (to a sixteenth)
+// for which all sequences' ranges fit the units: the longest work-group, and
+// with it the call, gets as short as the chip allows. Lane s computes
+// sequence s (at most 64); every wave that asks gets the same answer. u < 0:
+// the unit of range 0 of sequence `seq`.
+struct PrefillUnit {
+  int seq, first, ranges;
+};
+__device__ inline PrefillUnit prefill_unit(const PrefillArgs& a, int u, int seq, int lane) {
+  const int64_t p0 = lane < a.n_seqs ? (a.start_pos ? (int64_t)a.start_pos[lane] : a.p0) : 0;
+  const int st = lane < a.n_seqs ? prefill_steps(a, p0) : 0;
+  auto sum = [&](int v) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
+    return v;
+  };
+  int c = (sum(st) + a.units - 1) / a.units;
+  if (c < kPfMinSteps) c = kPfMinSteps;
+  int n = (st + c - 1) / c;
+  while (sum(n) > a.units) {  // ends: at c >= every st a sequence has one range, n_seqs <= units
+    c += 1 + c / 16;
+    n = (st + c - 1) / c;
+  }
+  int upto = n;  // units of sequences 0 .. lane
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    const int v = __shfl_up(upto, m);
+    if (lane >= m) upto += v;
+  }
+  PrefillUnit r;
+  if (u >= 0) {
+    const uint64_t past = __ballot(upto > u);
+    seq = past ? __builtin_ctzll(past) : -1;  // -1: a unit that nothing needs
+  }
+  r.seq = __builtin_amdgcn_readfirstlane(seq);
+  const int s = r.seq < 0 ? 0 : r.seq;
+  r.ranges = __builtin_amdgcn_readlane(n, s);
+  r.first = __builtin_amdgcn_readlane(upto, s) - r.ranges;
+  return r;
 }
 
 template <int D, int BITS, int MODE>
@@ -182,14 +281,20 @@ void prefill_attn_kernel(PrefillArgs a) {
   constexpr int CB = MODE == kCodebook ? BITS : 2;
 
   __shared__ __align__(16) uint8_t region[P::kRegion];
-  __shared__ float lrow[kPfRows];
+  __shared__ float lrow[kPfRows], mrow[kPfRows];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane >> 4, c = lane & 15;
   const int G = a.group;
   const int QP = kPfRows / G;  // query positions per work-group
-  const int kvh = blockIdx.y, seq = blockIdx.z;
+  const int kvh = blockIdx.y;
+  int seq = blockIdx.z, range = 0, ranges = 1;
+  if (a.units > 0) {
+    const PrefillUnit un = prefill_unit(a, blockIdx.z, 0, lane);
+    if (un.seq < 0) return;
+    seq = un.seq, range = (int)blockIdx.z - un.first, ranges = un.ranges;
+  }
   const int qi0 = blockIdx.x * QP;
   // paged: the sequence's start, through a scalar load (everything derived
   // from it stays in scalar registers)
@@ -289,44 +394,56 @@ void prefill_attn_kernel(PrefillArgs a) {
   float* const qsum = reinterpret_cast<float*>(qlo + kPfRows * QS);  // [row][NG] (affine)
   const uint32_t sbits = lane_sign_bits<D>(a.sign_bits, lane);
   const float cs_lane = fwht_lane_sign(lane) * a.c;
-#pragma unroll 2
-  for (int k = 0; k < kPfRows / NW; k++) {
-    const int r = wave + NW * k;
-    const int rq_ = r / G, rh_ = r - (r / G) * G;
-    const uint16_t* const src =
-        a.q + (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D +
-        lane * E;
-    if constexpr (MODE == kPlain) {
-      // E consecutive bf16 of the row as stored (zero past the chunk)
-      uint16_t* dst = reinterpret_cast<uint16_t*>(qhi + r * QS + lane * E);
+  // (eight rows' loads in flight together: one after the other, their latency
+  // made a 107-token chunk of head_dim 128, 32 rows a wave, twice as slow)
+#pragma unroll 1
+  for (int k0 = 0; k0 < kPfRows / NW; k0 += 8) {
+    uint32_t raw[8][E / 2];
 #pragma unroll
-      for (int i = 0; i < E; i++) dst[i] = rq_ < nq ? src[i] : (uint16_t)0;
-      continue;
+    for (int k = 0; k < 8; k++) {
+      const int r = wave + NW * (k0 + k);
+      const int rq_ = r / G, rh_ = r - rq_ * G;
+      const int64_t qi = qi0 + (rq_ < nq ? rq_ : 0);
+      load_words<E / 2>(
+          a.q + (((int64_t)seq * a.n_q + qi) * a.n_q_heads + (int64_t)kvh * G + rh_) * D + lane * E,
+          raw[k]);
+      if (rq_ >= nq) {  // zero past the chunk
+#pragma unroll
+        for (int i = 0; i < E / 2; i++) raw[k][i] = 0;
+      }
     }
-    float x[E];
 #pragma unroll
-    for (int i = 0; i < E; i++) x[i] = 0.0f;
-    if (rq_ < nq) {
-      load_row<E>(src, x);
+    for (int k = 0; k < 8; k++) {
+      const int r = wave + NW * (k0 + k);
+      if constexpr (MODE == kPlain) {
+        uint32_t* dst = reinterpret_cast<uint32_t*>(qhi + r * QS + lane * E);
 #pragma unroll
-      for (int i = 0; i < E; i++) x[i] = x[i] * a.qscale;
+        for (int i = 0; i < E / 2; i++) dst[i] = raw[k][i];
+        continue;
+      }
+      float x[E];
+#pragma unroll
+      for (int i = 0; i < E / 2; i++) {
+        x[2 * i] = __uint_as_float(raw[k][i] << 16) * a.qscale;
+        x[2 * i + 1] = __uint_as_float(raw[k][i] & 0xffff0000u) * a.qscale;
+      }
+      // the sign-tracking FWHT: a -0 for +0 changes no score or sum
+      wave_fwht_signed<E>(x, lane);
+      float gs = 0.0f;
+      _Float16 hv[E], lv[E];
+#pragma unroll
+      for (int i = 0; i < E; i++) {
+        const float v = apply_sign(x[i] * cs_lane, sbits, i);
+        gs += v;
+        hv[i] = (_Float16)v;
+        lv[i] = (_Float16)(v - (float)hv[i]);
+      }
+      gs = group_sum<LPG>(gs, lane);
+      store_halves<E>(reinterpret_cast<uint8_t*>(qhi + r * QS + lane * E), hv);
+      store_halves<E>(reinterpret_cast<uint8_t*>(qlo + r * QS + lane * E), lv);
+      if constexpr (MODE == kAffine)
+        if ((lane & (LPG - 1)) == 0) qsum[r * NG + ((lane * E) >> 6)] = gs;
     }
-    // the sign-tracking FWHT: a -0 for +0 changes no score or sum
-    wave_fwht_signed<E>(x, lane);
-    float gs = 0.0f;
-    _Float16 hv[E], lv[E];
-#pragma unroll
-    for (int i = 0; i < E; i++) {
-      const float v = apply_sign(x[i] * cs_lane, sbits, i);
-      gs += v;
-      hv[i] = (_Float16)v;
-      lv[i] = (_Float16)(v - (float)hv[i]);
-    }
-    gs = group_sum<LPG>(gs, lane);
-    store_halves<E>(reinterpret_cast<uint8_t*>(qhi + r * QS + lane * E), hv);
-    store_halves<E>(reinterpret_cast<uint8_t*>(qlo + r * QS + lane * E), lv);
-    if constexpr (MODE == kAffine)
-      if ((lane & (LPG - 1)) == 0) qsum[r * NG + ((lane * E) >> 6)] = gs;
   }
   __syncthreads();
 
@@ -599,7 +716,7 @@ void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             s[t][i] = s[t][i] * (ks[i] * cu);
-            vscale[t][i] = vs[i] * cu;
+            vscale[t][i] = vs[i] * (cu * kPvScale<CB>);
           }
         }
       } else if constexpr (MODE == kPlain) {
@@ -769,9 +886,11 @@ void prefill_attn_kernel(PrefillArgs a) {
     }
   };
 
-  // ---- the pipeline over steps s_begin .. s_end - 1 ----
-  const int s_begin = 0, s_end = nst;
-  const int n = s_end - s_begin;
+  // ---- the pipeline over the n steps from s_begin on ----
+  // (with several ranges, this one's share; possibly none)
+  const int per = ranges > 1 ? (nst + ranges - 1) / ranges : nst;
+  const int s_begin = range * per < nst ? range * per : nst;
+  const int n = nst - s_begin < per ? nst - s_begin : per;
   gptr_t cur[2], nxt[2], after[2];  // the blocks of steps i, i + 1, i + 2
   bool f_cur = false, f_nxt = false, f_after = false;
   // the blocks of step s_begin + i (past the end: of the last one)
@@ -839,7 +958,7 @@ void prefill_attn_kernel(PrefillArgs a) {
     if constexpr (!kOwn) l_run[u] += row_ror8(l_run[u]);
     l_run[u] = xor16_sum(l_run[u]);
     l_run[u] = xor32_sum(l_run[u]);
-    if (kOwn ? j == 0 : lane < 8) lrow[sm_row(u)] = l_run[u];
+    if (kOwn ? j == 0 : lane < 8) lrow[sm_row(u)] = l_run[u], mrow[sm_row(u)] = m_run[u];
   }
   lds_barrier();  // the buffers are free
   float* const Rr = reinterpret_cast<float*>(region);
@@ -849,49 +968,157 @@ void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
     for (int ct = 0; ct < 4; ct++)
       *reinterpret_cast<float4_t*>(&Rr[(rt * 16 + c) * RS + wave * 64 + ct * 16 + 4 * j]) =
-          MODE == kAffine ? o[rt][ct] + bacc[rt] : o[rt][ct];
+          MODE == kAffine     ? o[rt][ct] + bacc[rt]
+          : MODE == kCodebook ? o[rt][ct] * (1.0f / kPvScale<CB>)
+                              : o[rt][ct];
   }
   __syncthreads();
+  if (ranges > 1) {  // partial rows, as accumulated, with their (m, l)
+    const int64_t slot =
+        (((int64_t)blockIdx.z * gridDim.y + kvh) * gridDim.x + blockIdx.x) * kPfRows;
 #pragma unroll 2
-  for (int k = 0; k < kPfRows / NW; k++) {
-    const int r = wave + NW * k;
-    const int rq_ = r / G, rh_ = r - (r / G) * G;
-    if (rq_ >= nq) continue;
-    const float l = lrow[r];
-    float x[E];
-    float cs = cs_lane;
-    if constexpr (MODE != kPlain) {
+    for (int k = 0; k < kPfRows / NW; k++) {
+      const int r = wave + NW * k;
+      float* dst = a.part_o + (slot + r) * D + lane * E;
 #pragma unroll
-      for (int i = 0; i < E; i++) x[i] = apply_sign(Rr[r * RS + lane * E + i], sbits, i);
+      for (int i = 0; i < E; i++) dst[i] = Rr[r * RS + lane * E + i];
+    }
+    if (tid < kPfRows)
+      *reinterpret_cast<float2*>(a.part_ml + (slot + tid) * 2) = make_float2(mrow[tid], lrow[tid]);
+    return;
+  }
+#pragma unroll 1
+  for (int k0 = 0; k0 < kPfRows / NW; k0 += 4) {
+    float x[4][E];  // four rows at a time, past the chunk too (not stored)
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int r = wave + NW * (k0 + k);
+#pragma unroll
+      for (int i = 0; i < E; i++) x[k][i] = Rr[r * RS + lane * E + i];
+      if constexpr (MODE != kPlain) {  // (plain: no rotation, the row as accumulated)
+#pragma unroll
+        for (int i = 0; i < E; i++) x[k][i] = apply_sign(x[k][i], sbits, i);
+        wave_fwht_signed<E>(x[k], lane);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int r = wave + NW * (k0 + k);
+      const int rq_ = r / G, rh_ = r - rq_ * G;
+      if (rq_ >= nq) continue;
+      const float l = lrow[r];
+#pragma unroll
+      for (int i = 0; i < E; i++)
+        x[k][i] = l > 0.0f ? (x[k][i] * (MODE == kPlain ? 1.0f : cs_lane)) / l : 0.0f;
+      store_out<E>(a, (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D +
+                          lane * E, x[k]);
+    }
+  }
+}
+
+// Merges the key ranges of a split sequence's rows: a wave per row, lane l
+// holding dims E l .., out = sum_k 2^(m_k - M) O_k / sum_k 2^(m_k - M) l_k,
+// rotated back. Reads each partial once (bound by that: D * 4 bytes a row and
+// range). A work-group takes 16 rows of a tile.
+constexpr int kPfMergeRows = 16;
+template <int D, bool ROT>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int tiles) {
+  constexpr int E = D / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int seq = blockIdx.z, kvh = blockIdx.y;
+  const int tile = blockIdx.x / (kPfRows / kPfMergeRows);
+  const int r0 = (blockIdx.x % (kPfRows / kPfMergeRows)) * kPfMergeRows;
+  const PrefillUnit un = prefill_unit(a, -1, seq, lane);
+  if (un.ranges <= 1) return;
+  const int G = a.group, QP = kPfRows / G;
+  const int nq = a.n_q - tile * QP < QP ? a.n_q - tile * QP : QP;
+  const uint32_t sbits = lane_sign_bits<D>(a.sign_bits, lane);
+  const float cs = ROT ? fwht_lane_sign(lane) * a.c : 1.0f;
+#pragma unroll 1
+  for (int r = r0 + wave; r < r0 + kPfMergeRows; r += 4) {
+    const int rq = r / G, rh = r - rq * G;
+    if (rq >= nq) break;
+    const int64_t step = (int64_t)gridDim.y * tiles * kPfRows;  // rows from range to range
+    const int64_t row = (((int64_t)un.first * gridDim.y + kvh) * tiles + tile) * kPfRows + r;
+    float M = -1e30f;
+    for (int k = lane; k < un.ranges; k += 64) M = fmaxf(M, a.part_ml[(row + k * step) * 2]);
+    M = group_max<64>(M, lane);
+    float x[E], l = 0.0f;
+#pragma unroll
+    for (int i = 0; i < E; i++) x[i] = 0.0f;
+#pragma unroll 2
+    for (int k = 0; k < un.ranges; k++) {
+      const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + (row + k * step) * 2);
+      const float w = __builtin_amdgcn_exp2f(ml.x - M);
+      const float* src = a.part_o + (row + k * step) * D + lane * E;
+      l = fmaf(w, ml.y, l);
+#pragma unroll
+      for (int i = 0; i < E; i++) x[i] = fmaf(w, src[i], x[i]);
+    }
+    if constexpr (ROT) {
+#pragma unroll
+      for (int i = 0; i < E; i++) x[i] = apply_sign(x[i], sbits, i);
       wave_fwht_signed<E>(x, lane);
-    } else {  // no rotation: the row as accumulated
-#pragma unroll
-      for (int i = 0; i < E; i++) x[i] = Rr[r * RS + lane * E + i];
-      cs = 1.0f;
     }
-    const int64_t o_idx =
-        (((int64_t)seq * a.n_q + qi0 + rq_) * a.n_q_heads + (int64_t)kvh * G + rh_) * D + lane * E;
 #pragma unroll
-    for (int i = 0; i < E; i++) {
-      const float v = l > 0.0f ? (x[i] * cs) / l : 0.0f;
-      if (a.out_f32)
-        reinterpret_cast<float*>(a.out)[o_idx + i] = v;
-      else
-        reinterpret_cast<uint16_t*>(a.out)[o_idx + i] = f32_to_bf16(v);
-    }
+    for (int i = 0; i < E; i++) x[i] = l > 0.0f ? (x[i] * cs) / l : 0.0f;
+    store_out<E>(a, (((int64_t)seq * a.n_q + tile * QP + rq) * a.n_q_heads + (int64_t)kvh * G + rh) * D +
+                        lane * E, x);
   }
 }
 
 template <int D, int BITS, int MODE>
 hipError_t launch_t(const PrefillArgs& a, hipStream_t s) {
   const int qp = kPfRows / a.group;
-  dim3 grid((a.n_q + qp - 1) / qp, a.new_st.n_kv_heads, a.n_seqs);
+  const int tiles = (a.n_q + qp - 1) / qp, H = a.new_st.n_kv_heads;
+  dim3 grid(tiles, H, a.units > 0 ? a.units : a.n_seqs);
   hipLaunchKernelGGL((prefill_attn_kernel<D, BITS, MODE>), grid,
                      dim3(PfPlan<D, BITS, MODE>::NW * 64), 0, s, a);
+  if (a.units > 0) {
+    dim3 mgrid(tiles * (kPfRows / kPfMergeRows), H, a.n_seqs);
+    hipLaunchKernelGGL((prefill_merge_kernel<D, MODE != kPlain>), mgrid, dim3(256), 0, s, a, tiles);
+  }
   return hipGetLastError();
 }
 
 }  // namespace
+
+// Short contexts go to fmkv_prefill_short.hip, up to where its time (first)
+// crosses this file's: 4-bit affine, 107 tokens after 50 (7 steps): 27 / 44 us
+// at head_dim 128, 34 / 39 at 256, 51 / 46 at 512; 4 x 300 after 200 (17
+// steps): 55 / 63, 117 / 96; 2 x 3 after 64 (4 steps): 18 / 33, 21 / 30, 32 /
+// 37; 20 after 400 (15 steps, split): 49 / 43, 59 / 42. Plain caches rotate
+// nothing: 2 x 3 after 64: 16 / 21, 18 / 19, 26 / 23; 107 after 50: 25 / 33,
+// 34 / 30.
+bool prefill_is_short(const PrefillArgs& a, int64_t max_steps) {
+  const int D = a.new_st.layout.head_dim;
+  if (a.new_st.layout.mode == kPlain) return max_steps <= (D == 128 ? 8 : D == 256 ? 4 : 0);
+  if (D == 128) {
+    // (few rows: the split of a longer context pays earlier)
+    const int64_t rows = (int64_t)a.n_seqs * a.n_q * a.n_q_heads;
+    return max_steps <= (rows >= 1024 ? 20 : 12);
+  }
+  return max_steps <= (D == 256 ? 8 : 4);
+}
+
+// The units of a split call (0: not split), and the bytes of its partials.
+// Worth it when one work-group per (tile, KV head, sequence) leaves at least
+// a whole round of CUs' places unused, so that the units all run at once, and
+// some sequence is long enough for two ranges. Work-groups per CU: the waves
+// that the registers of a SIMD hold, two, times four.
+int prefill_units(const PrefillArgs& a, int cus, int64_t max_steps, size_t* bytes) {
+  const int D = a.new_st.layout.head_dim, qp = kPfRows / a.group;
+  const int64_t wgs = (int64_t)((a.n_q + qp - 1) / qp) * a.new_st.n_kv_heads;  // per unit
+  const int64_t places = (int64_t)cus * (D == 512 ? 1 : D == 256 ? 2 : 3);
+  *bytes = 0;
+  if (a.n_seqs > 64 || max_steps < 2 * kPfMinSteps) return 0;
+  int64_t units = places / wgs;
+  const int64_t most = a.n_seqs * ((max_steps + kPfMinSteps - 1) / kPfMinSteps);
+  if (units > most) units = most;
+  if (units <= a.n_seqs) return 0;
+  *bytes = (size_t)(units * wgs * kPfRows) * (D + 2) * sizeof(float);
+  return (int)units;
+}
 
 hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t s) {
   if (a.n_q <= 0) return hipSuccess;

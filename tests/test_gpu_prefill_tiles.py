@@ -41,7 +41,7 @@ def test_prefill_tile_edges(gpu, ora, mode, D, bits, Hkv, Hq, window):
 
     tile = 64 // (Hq // Hkv)
     for prefix, n in ((0, 1), (0, tile + 1), (15, tile), (16, tile - 1 or 1), (31, 17), (33, tile + 1),
-                      (300, 2 * tile + 1)):
+                      (300, 2 * tile + 1), (640, tile), (655, tile + 1), (672, 1), (687, 17)):
         cap = 0 if window else prefix + n
         if mode == 2:
             cache = gpu.KVCache.new_with_window(D, window or None, Hkv, cap)
@@ -59,3 +59,69 @@ def test_prefill_tile_edges(gpu, ora, mode, D, bits, Hkv, Hq, window):
         torch.cuda.synchronize()
         err = np.abs(out.cpu().numpy().astype(np.float64) - oc.prefill(k, v, q, scale))
         assert err.max() < 4e-3 and err.mean() < 1.2e-4, f"prefix {prefix} n {n}: {err.max():.2e} {err.mean():.2e}"
+
+
+@pytest.mark.parametrize("mode,D,bits,Hq", [(0, 512, 8, 8), (1, 256, 3, 4), (2, 128, 16, 8)])
+def test_prefill_split_ragged_and_captured(gpu, ora, mode, D, bits, Hq):
+    """A few rows of ragged sequences (one too short for a second key range,
+    one long, one that starts at its chunk), split over the keys; twice in a
+    row, then on a second stream right after the first, then captured (there
+    unsplit) and replayed: the oracle's result each time; the same bits from every split call."""
+    import torch
+
+    starts, n, Hkv = [20, 1500, 0, 333], 5, 1
+    need = [(p + n + 15) // 16 for p in starts]
+    table = np.zeros((len(starts), max(need)), np.int32)
+    at = 0
+    for s, nb in enumerate(need):
+        table[s, :nb] = np.arange(at, at + nb)[::-1]
+        at += nb
+    pool = gpu.PagedPool(gpu.make_desc(Hkv, D, bits, mode=mode), at)
+    dtab = torch.from_numpy(table).cuda()
+    dstart = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    k, v = kv_batch(1, len(starts) * n, Hkv, D), kv_batch(2, len(starts) * n, Hkv, D)
+    q = soft_q(3, len(starts) * n, Hq, D)
+    shape = (len(starts), n, -1, D)
+    k, v, q = k.reshape(shape), v.reshape(shape), q.reshape(shape)
+    scale = 0.3 / np.sqrt(D)
+    want = []
+    for s, p in enumerate(starts):
+        oc = ora.OracleCache(Hkv, D, bits, 0, p + n, mode=mode)
+        if p:
+            k0, v0 = kv_batch(10 + s, p, Hkv, D), kv_batch(20 + s, p, Hkv, D)
+            oc.append(k0, v0)
+            pool.append(dev_bf16(k0)[None], dev_bf16(v0)[None], dtab[s:s + 1],
+                        torch.zeros(1, dtype=torch.int32, device="cuda"))
+        want.append(oc.prefill(k[s], v[s], q[s], scale))
+    want = np.stack(want)
+    dk, dv, dq = dev_bf16(k), dev_bf16(v), dev_bf16(q)
+
+    def call():
+        return pool.prefill_step(dk, dv, dtab, dstart, dq, scale, dtype=torch.float32)
+
+    def check(out, what):
+        err = np.abs(out.cpu().numpy().astype(np.float64) - want)
+        # (a codebook row's reconstruction is not bounded by its largest value,
+        # as the bound above takes it: the path's own 2e-2 for the worst value,
+        # the mean bound as above)
+        assert err.max() < 2e-2 and err.mean() < 1.2e-4, f"{what}: {err.max():.2e} {err.mean():.2e}"
+
+    first, second = call(), call()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    third = call()
+    with torch.cuda.stream(side):
+        fourth = call()
+    torch.cuda.synchronize()
+    check(first, "split")
+    for o in (second, third, fourth):
+        assert torch.equal(first, o)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        captured = call()
+    for i in range(3):
+        captured.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        check(captured, f"replay {i}")
+        assert torch.equal(first, call())
