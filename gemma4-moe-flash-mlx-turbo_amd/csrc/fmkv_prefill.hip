@@ -179,12 +179,14 @@ __device__ inline T load_at(gptr_t p, uint32_t off) {
   return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off);
 }
 
+// 2 N consecutive bf16 in one load a lane (aligned to one of them only).
 template <int N>
 __device__ inline void load_words(const uint16_t* src, uint32_t (&w)[N]) {
-  typedef uint32_t vec __attribute__((ext_vector_type(N == 1 ? 2 : N)));
   if constexpr (N == 1) {
-    w[0] = *reinterpret_cast<const uint32_t*>(src);
+    typedef uint32_t word __attribute__((aligned(2)));
+    w[0] = *reinterpret_cast<const word*>(src);
   } else {
+    typedef uint32_t vec __attribute__((ext_vector_type(N), aligned(2)));
     const vec v = *reinterpret_cast<const vec*>(src);
 #pragma unroll
     for (int i = 0; i < N; i++) w[i] = v[i];
