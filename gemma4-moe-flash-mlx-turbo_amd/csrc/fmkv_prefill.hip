@@ -218,6 +218,14 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// From here on a finite f16 result that overflows is 65504 and not infinity
+// (MODE.FP16_OVFL, this wave only): a weight P' of more than 65504 -- p up to
+// 2^8 times a V scale (affine) or norm / sqrt(D) (4-bit codebook) of 256 and
+// more -- is then 65504 and a residual of up to as much, and no Inf - Inf.
+__device__ inline void f16_overflow_saturates() {
+  __builtin_amdgcn_s_setreg(1 | (23 << 6), 1);  // hwreg MODE (1), bit 23, one bit
+}
+
 // Steps (32 keys) that a row tile of a sequence may need, from its start.
 __device__ inline int prefill_steps(const PrefillArgs& a, int64_t p0) {
   const int64_t lo = a.vis_begin > 0 ? a.vis_begin : 0;
@@ -284,6 +292,8 @@ void prefill_attn_kernel(PrefillArgs a) {
 
   __shared__ __align__(16) uint8_t region[P::kRegion];
   __shared__ float lrow[kPfRows], mrow[kPfRows];
+
+  f16_overflow_saturates();
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -848,8 +858,9 @@ void prefill_attn_kernel(PrefillArgs a) {
       const u32x4 w1 = pb[buf * (P::kPb / 16) + (j + 4) * kPfRows + rt * 16 + c];
       half8_t bh, bl;
       if constexpr (MODE == kAffine) {
-        // P' = p * v_scale in packed f16: the high part P_hi * s rounded, then
-        // its exact rounding error plus P_lo * s
+        // P' = p * v_scale in packed f16: the high part P_hi * s rounded (or
+        // 65504), then what that left out plus P_lo * s, rounded in turn (its
+        // grid ends at 2^-24)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const half2_t ph = __builtin_bit_cast(half2_t, e < 2 ? w0[e] : w1[e - 2]);

@@ -125,3 +125,51 @@ def test_prefill_split_ragged_and_captured(gpu, ora, mode, D, bits, Hq):
         torch.cuda.synchronize()
         check(captured, f"replay {i}")
         assert torch.equal(first, call())
+
+
+@pytest.mark.parametrize("mode,D,bits,Hq,amp", [
+    (0, 512, 4, 8, 3700.0), (0, 256, 4, 4, 3700.0), (0, 128, 4, 2, 3700.0), (0, 512, 8, 8, 62000.0),
+    (0, 128, 8, 4, 62000.0), (1, 512, 4, 8, 450.0), (1, 256, 4, 2, 450.0), (1, 128, 4, 4, 450.0)])
+@pytest.mark.parametrize("n", [5, 600])
+def test_prefill_weights_beyond_f16(gpu, ora, mode, D, bits, Hq, amp, n):
+    """V scales of up to 511 (affine) and norms / sqrt(D) of 450 (4-bit
+    codebook) behind scores that rise by 7.75 (base 2) after the first keys,
+    less than what moves the reference maximum: weights p * scale of up to
+    1.1e5, past f16's 65504, where the pair is 65504 and a residual r <= 65504
+    rounded to 2^-11 of itself, hence good to 2^-12 of the weight and the
+    value to 2^-12 of the longest row that it averages."""
+    import torch
+
+    prefix, Hkv = 700, 1
+    cap = prefix + n
+    rng = np.random.default_rng(n + D)
+
+    def bf16(x):
+        return (np.ascontiguousarray(x, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+    u = rng.standard_normal(D).astype(np.float32)
+    k = np.tile(u, (cap, Hkv, 1))
+    k[:48] = 0.0
+    oc = ora.OracleCache(Hkv, D, bits, 0, cap, mode=mode)
+    if mode == 0:  # uniform in the stored basis: scale = range / codes, biases within f16
+        y = rng.uniform(-1.0, 1.0, (cap, Hkv, D)) * rng.uniform(0.65 * amp, amp, (cap, 1, 1))
+        v = ora.unrotate_rows_f64(y, oc.sgn)
+    else:  # rows of one norm
+        v = rng.standard_normal((cap, Hkv, D))
+        v *= amp * np.sqrt(D) / np.linalg.norm(v, axis=-1, keepdims=True)
+    k, v, q = bf16(k), bf16(v), np.tile(bf16(u), (n, Hq, 1))
+    oc.append(k[:prefix], v[:prefix])
+    ks, vs = oc.dequant_kv()
+    score = float(ks[-1, 0] @ (q[0, 0].astype(np.uint32) << 16).view(np.float32))
+    scale = float(np.float32(7.75 * np.log(2.0) / score))
+    held = oc.meta[:prefix, 1, 0].view(np.float16).astype(np.float64)
+    held = np.abs(held[:, 0::2]) if mode == 0 else held / np.sqrt(D)
+    assert 65520 < 2.0 ** 7.75 * held.max() < 131008 and held.max() < 511
+    cache = gpu.KVCache(gpu.make_desc(Hkv, D, bits, 0, cap, mode))
+    cache.append(dev_bf16(k[:prefix]), dev_bf16(v[:prefix]))
+    out = cache.prefill_step(dev_bf16(k[prefix:]), dev_bf16(v[prefix:]), dev_bf16(q), scale,
+                             dtype=torch.float32)
+    torch.cuda.synchronize()
+    err = np.abs(out.cpu().numpy().astype(np.float64) - oc.prefill(k[prefix:], v[prefix:], q, scale))
+    bound = 2.0 ** -12 * np.sqrt((vs ** 2).sum(-1).max())
+    assert np.isfinite(err).all() and err.max() < bound, f"{err.max():.3e} of {bound:.3e}"
