@@ -82,6 +82,8 @@
 // positions early queries still need), the rest from new_st (a staging
 // copy of the chunk, or the cache itself for linear caches). A block that
 // straddles p_split is visited once per store with the other part masked.
+#include <type_traits>
+
 #include "fmkv_device.h"
 #include "fmkv_internal.h"
 #include "fmkv_attn_common.h"
@@ -95,11 +97,18 @@ constexpr int kPfTiles = kPfRows / 16;
 constexpr int kPfKeys = 2 * kBlockTokens;  // keys per step
 constexpr int kPfQuads = kPfKeys / 4;      // groups of four keys of a step
 constexpr int kPfMinSteps = 4;             // steps of the shortest key range of a split call
+// How far (base 2) a score may exceed its row's reference maximum before the
+// row is rescaled. Weights stay below 2^7, and a weight times a V scale that an
+// affine cache's attention documents as valid (below 511) within f16. The
+// matrix cores would take an infinite high part and residual to NaN. (MODE's
+// FP16_OVFL clamps such results to 65504 at no cost, but the matrix cores heed
+// it too and turn infinite products and sums into finite ones.)
+constexpr float kPfSlack = 7.0f;
 
 // 2- and 3-bit codebook caches weigh V by p * norm / (1000 sqrt(D)), mostly
 // below 2^-8, where an f16 residual is subnormal and ends at 2^-25: their
 // weights carry a factor 32 that the accumulated row loses again (norm is an
-// f16, so p <= 2^8 and D >= 128 keep them below 4.8e4). Error against 64 bits
+// f16, so p <= 2^7 and D >= 128 keep them below 2.4e4). Error against 64 bits
 // over 6000 positions: 1.8e-4 without it.
 template <int BITS>
 constexpr float kPvScale = kCbExact<BITS> ? 32.0f : 1.0f;
@@ -174,8 +183,12 @@ __device__ inline uint32_t pack_bf16x2(float a, float b) {
 typedef const uint8_t __attribute__((address_space(1)))* gptr_t;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x2 u32x2_a4 __attribute__((aligned(4)));  // two words at a 4-byte boundary
+// The offset is opaque where it is used, or its extension to 64 bits leaves the
+// loop, and with it the form of the load that adds a 32-bit one to a scalar
+// base: 8 registers and 8 additions a step in a loop that is short of both.
 template <class T>
 __device__ inline T load_at(gptr_t p, uint32_t off) {
+  asm volatile("" : "+v"(off));
   return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off);
 }
 
@@ -216,14 +229,6 @@ __device__ inline void store_out(const PrefillArgs& a, int64_t o_idx, const floa
 // memory stay in flight across it.
 __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// From here on a finite f16 result that overflows is 65504 and not infinity
-// (MODE.FP16_OVFL, this wave only): a weight P' of more than 65504 -- p up to
-// 2^8 times a V scale (affine) or norm / sqrt(D) (4-bit codebook) of 256 and
-// more -- is then 65504 and a residual of up to as much, and no Inf - Inf.
-__device__ inline void f16_overflow_saturates() {
-  __builtin_amdgcn_s_setreg(1 | (23 << 6), 1);  // hwreg MODE (1), bit 23, one bit
 }
 
 // Steps (32 keys) that a row tile of a sequence may need, from its start.
@@ -292,8 +297,7 @@ void prefill_attn_kernel(PrefillArgs a) {
 
   __shared__ __align__(16) uint8_t region[P::kRegion];
   __shared__ float lrow[kPfRows], mrow[kPfRows];
-
-  f16_overflow_saturates();
+  __shared__ int not_finite;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -404,6 +408,7 @@ void prefill_attn_kernel(PrefillArgs a) {
   _Float16* const qhi = reinterpret_cast<_Float16*>(region);
   _Float16* const qlo = qhi + kPfRows * QS;
   float* const qsum = reinterpret_cast<float*>(qlo + kPfRows * QS);  // [row][NG] (affine)
+  if (tid == 0) not_finite = 0;
   const uint32_t sbits = lane_sign_bits<D>(a.sign_bits, lane);
   const float cs_lane = fwht_lane_sign(lane) * a.c;
   // (eight rows' loads in flight together: one after the other, their latency
@@ -691,7 +696,9 @@ void prefill_attn_kernel(PrefillArgs a) {
     }
   };
 
-  auto softmax = [&](int buf, int step, const float4_t (&mine)[NRS][2], bool full) __attribute__((always_inline)) {
+  // HIDE: as hide_not_finite
+  auto softmax = [&](int buf, int step, const float4_t (&mine)[NRS][2], bool full, auto hide) __attribute__((always_inline)) {
+    constexpr bool HIDE = decltype(hide)::value;
 #pragma unroll
     for (int u = 0; u < NRS; u++) {
       const int row = sm_row(u);
@@ -749,7 +756,10 @@ void prefill_attn_kernel(PrefillArgs a) {
           const int kp = (vi < n_old_i ? vi : vi + vb_shift) * kBlockTokens + 4 * (quad0 & 3);
 #pragma unroll
           for (int i = 0; i < 4; i++)
-            if (!(kp + i >= vlo && kp + i < vhi)) s[t][i] = -INFINITY;
+            if (!(kp + i >= vlo && kp + i < vhi)) {
+              s[t][i] = -INFINITY;
+              if constexpr (HIDE && MODE == kCodebook) vscale[t][i] = 0.0f;
+            }
         }
       }
       float mb = -INFINITY;
@@ -761,7 +771,7 @@ void prefill_attn_kernel(PrefillArgs a) {
       mb = xor32_max(mb);
       const float m_new = fmaxf(m_run[u], mb);
       const float m_old = m_run[u];
-      m_run[u] = __any(m_new > m_old + kRescaleSlack) ? m_new : m_old;
+      m_run[u] = __any(m_new > m_old + kPfSlack) ? m_new : m_old;
       const float alpha = __builtin_amdgcn_exp2f(m_old - m_run[u]);  // 1 when it stays
       l_run[u] *= alpha;
       if (kOwn ? j == 0 : lane < 8) al[buf * kPfRows + (row & 15) * 4 + (row >> 4)] = alpha;
@@ -783,8 +793,16 @@ void prefill_attn_kernel(PrefillArgs a) {
             // (one rounded product for both parts: fused into either conversion
             // it can round the high part to its other neighbour)
             asm("" : "+v"(x));
-            h[i] = (_Float16)x;
-            r[i] = (_Float16)(x - (float)h[i]);
+            if constexpr (MODE == kCodebook && !kCbExact<CB>) {
+              // (4 bits: norm / sqrt(D) has no bound. At most 65504 and a
+              // residual of as much, cut: infinite parts would meet as NaN.
+              // What is infinite or NaN before stays so, in the residual.)
+              h[i] = (_Float16)fminf(x, 65504.0f);
+              r[i] = pkrtz(x - (float)h[i], 0.0f)[0];
+            } else {
+              h[i] = (_Float16)x;
+              r[i] = (_Float16)(x - (float)h[i]);
+            }
           }
           const uint2 hw = __builtin_bit_cast(uint2, h), rw = __builtin_bit_cast(uint2, r);
           w = (u32x4){hw.x, hw.y, rw.x, rw.y};
@@ -812,7 +830,7 @@ void prefill_attn_kernel(PrefillArgs a) {
       }
     }
   };
-  auto pv = [&](int buf) __attribute__((always_inline)) {
+  auto pv = [&](int buf, auto hide) __attribute__((always_inline)) {
     half2_t vsc[4], vbi[4];  // affine: scales and biases of the lane's key pairs
     if constexpr (MODE == kAffine) {
 #pragma unroll
@@ -858,16 +876,23 @@ void prefill_attn_kernel(PrefillArgs a) {
       const u32x4 w1 = pb[buf * (P::kPb / 16) + (j + 4) * kPfRows + rt * 16 + c];
       half8_t bh, bl;
       if constexpr (MODE == kAffine) {
-        // P' = p * v_scale in packed f16: the high part P_hi * s rounded (or
-        // 65504), then what that left out plus P_lo * s, rounded in turn (its
-        // grid ends at 2^-24)
+        // P' = p * v_scale in packed f16: the high part P_hi * s rounded, then
+        // what that left out plus P_lo * s, rounded in turn (its grid ends at
+        // 2^-24). HIDE: from 32 bits, toward zero, so that a scale beyond the
+        // documented ones ends in 65504 and a residual of as much at most.
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const half2_t ph = __builtin_bit_cast(half2_t, e < 2 ? w0[e] : w1[e - 2]);
           const half2_t pl = __builtin_bit_cast(half2_t, e < 2 ? w0[e + 2] : w1[e]);
-          const half2_t h = ph * vsc[e];
-          const half2_t l = __builtin_elementwise_fma(
+          half2_t h = ph * vsc[e];
+          half2_t l = __builtin_elementwise_fma(
               pl, vsc[e], __builtin_elementwise_fma(ph, vsc[e], -h));
+          if constexpr (decltype(hide)::value) {
+            const float x0 = ((float)ph[0] + (float)pl[0]) * (float)vsc[e][0];
+            const float x1 = ((float)ph[1] + (float)pl[1]) * (float)vsc[e][1];
+            h = pkrtz(x0, x1);
+            l = pkrtz(x0 - (float)h[0], x1 - (float)h[1]);
+          }
           bh[2 * e] = h[0];
           bh[2 * e + 1] = h[1];
           bl[2 * e] = l[0];
@@ -896,6 +921,72 @@ void prefill_attn_kernel(PrefillArgs a) {
           o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[ct], bl, o[rt][ct], 0, 0, 0);
         }
       }
+    }
+  };
+
+  // V values (affine: scales and biases) that are not finite, in a step whose
+  // keys some rows do not see: a hidden key's weight 0 makes NaN of them. They
+  // become 0, and NaN the accumulators of the rows that do see them.
+  auto hide_not_finite = [&](int step) __attribute__((always_inline)) {
+    constexpr uint32_t kExp = MODE == kPlain ? 0x7f80u : 0x7c00u;
+    // all bits of the 16-bit values in w that are not finite
+    auto bad_of = [&](uint32_t w) __attribute__((always_inline)) -> uint32_t {
+      return ((w & kExp) == kExp ? 0xffffu : 0u) |
+             ((w & (kExp << 16)) == (kExp << 16) ? 0xffff0000u : 0u);
+    };
+    // bit 4 kt + i: row 16 rt + c sees the lane's key 4 j + i of block kt
+    auto seen_of = [&](int rt) __attribute__((always_inline)) -> uint32_t {
+      const int p = pA_r + (rt * 16 + c) / G;
+      uint32_t m = 0;
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++) {
+        const int vi = 2 * step + kt, lo = lo_rel(p);
+        int vlo, vhi;
+        vb_range(vi, vlo, vhi);
+        vlo = vlo > lo ? vlo : lo;
+        vhi = vhi < p + 1 ? vhi : p + 1;
+        const int kp = (vi < n_old_i ? vi : vi + vb_shift) * kBlockTokens + 4 * j;
+#pragma unroll
+        for (int i = 0; i < 4; i++) m |= kp + i >= vlo && kp + i < vhi ? 1u << (4 * kt + i) : 0u;
+      }
+      return m;
+    };
+    if constexpr (MODE == kPlain) {
+#pragma unroll
+      for (int rt = 0; rt < kPfTiles; rt++) {
+        // how many of them a row sees, per dim: a product of ones
+        const uint32_t m = seen_of(rt);
+        u32x4 seen;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          seen[e] = (m >> (2 * e) & 1 ? 0x3f80u : 0u) | (m >> (2 * e) & 2 ? 0x3f800000u : 0u);
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) {
+          u32x4 bad;
+#pragma unroll
+          for (int e = 0; e < 4; e++) bad[e] = bad_of(vr[e >> 1][2 * ct + (e & 1)]) & 0x3f803f80u;
+          const float4_t n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, bad), __builtin_bit_cast(bf16x8_t, seen),
+              (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; i++) o[rt][ct][i] = n[i] > 0.0f ? NAN : o[rt][ct][i];
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < VW; w++) {
+        vr[0][w] &= ~bad_of(vr[0][w]);
+        vr[1][w] &= ~bad_of(vr[1][w]);
+      }
+    } else if constexpr (MODE == kAffine) {
+      uint32_t bad = 0;
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        bad |= bad_of(vm[b >> 2][b & 3]) ? 1u << b : 0u;
+        vm[b >> 2][b & 3] = bad >> b & 1 ? 0u : vm[b >> 2][b & 3];
+      }
+#pragma unroll
+      for (int rt = 0; rt < kPfTiles; rt++)  // (the lanes' sums join the row at the end)
+        bacc[rt] = bad & seen_of(rt) ? NAN : bacc[rt];
     }
   };
 
@@ -953,16 +1044,61 @@ void prefill_attn_kernel(PrefillArgs a) {
       rescale((i - 1) & 1);
       qk((i + 1) & 1);
       load_k(after);
-      softmax(i & 1, s_begin + i, mine, f_cur);
+      softmax(i & 1, s_begin + i, mine, f_cur, std::false_type{});
       keep_own();
       load_n(nxt);
-      pv((i - 1) & 1);
+      pv((i - 1) & 1, std::false_type{});
       load_v(cur);
       lds_barrier();
       advance(i + 1);
     }
     rescale((n - 1) & 1);
-    pv((n - 1) & 1);
+    pv((n - 1) & 1, std::false_type{});
+  }
+
+  // A sum that is not finite: some V value was not (or some score), and a row
+  // that does not see it may have it all the same, as 0 * inf; or a V scale
+  // took a weight past f16. The steps again, one stage after the other, with
+  // such values kept from those rows and such weights saturated. (Tested here
+  // and not where V is read: a test in the steps with hidden keys alone cost
+  // 2% of every call.)
+  bool bad = false;
+#pragma unroll
+  for (int rt = 0; rt < kPfTiles; rt++) {
+    float s = MODE == kAffine ? bacc[rt] * 0.0f : 0.0f;
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) s = fmaf(o[rt][ct][i], 0.0f, s);
+    bad = bad || s != 0.0f;
+  }
+  if (__any(bad)) not_finite = 1;
+  lds_barrier();  // the buffers are free
+  if (not_finite) {
+#pragma unroll
+    for (int rt = 0; rt < kPfTiles; rt++) {
+      bacc[rt] = 0.0f;
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) o[rt][ct] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int u = 0; u < NRS; u++) m_run[u] = -1e30f, l_run[u] = 0.0f;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+      blocks_of(i, cur, f_cur);
+      load_k(cur);
+      load_n(cur);
+      load_v(cur);
+      qk(0);
+      keep_own();
+      lds_barrier();
+      softmax(0, s_begin + i, mine, f_cur, std::true_type{});
+      lds_barrier();
+      rescale(0);
+      if (!f_cur) hide_not_finite(s_begin + i);
+      pv(0, std::true_type{});
+    }
+    lds_barrier();
   }
 
   // ---- epilogue: normalise, inverse rotation, store ----
@@ -973,7 +1109,6 @@ void prefill_attn_kernel(PrefillArgs a) {
     l_run[u] = xor32_sum(l_run[u]);
     if (kOwn ? j == 0 : lane < 8) lrow[sm_row(u)] = l_run[u], mrow[sm_row(u)] = m_run[u];
   }
-  lds_barrier();  // the buffers are free
   float* const Rr = reinterpret_cast<float*>(region);
 #pragma unroll
   for (int rt = 0; rt < kPfTiles; rt++) {

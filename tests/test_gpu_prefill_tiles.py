@@ -129,15 +129,18 @@ def test_prefill_split_ragged_and_captured(gpu, ora, mode, D, bits, Hq):
 
 @pytest.mark.parametrize("mode,D,bits,Hq,amp", [
     (0, 512, 4, 8, 3700.0), (0, 256, 4, 4, 3700.0), (0, 128, 4, 2, 3700.0), (0, 512, 8, 8, 62000.0),
-    (0, 128, 8, 4, 62000.0), (1, 512, 4, 8, 450.0), (1, 256, 4, 2, 450.0), (1, 128, 4, 4, 450.0)])
-@pytest.mark.parametrize("n", [5, 600])
-def test_prefill_weights_beyond_f16(gpu, ora, mode, D, bits, Hq, amp, n):
-    """V scales of up to 511 (affine) and norms / sqrt(D) of 450 (4-bit
-    codebook) behind scores that rise by 7.75 (base 2) after the first keys,
-    less than what moves the reference maximum: weights p * scale of up to
-    1.1e5, past f16's 65504, where the pair is 65504 and a residual r <= 65504
-    rounded to 2^-11 of itself, hence good to 2^-12 of the weight and the
-    value to 2^-12 of the longest row that it averages."""
+    (0, 128, 8, 4, 62000.0), (1, 512, 4, 8, 450.0), (1, 256, 4, 2, 450.0), (1, 128, 4, 4, 450.0),
+    (0, 512, 4, 8, 7500.0), (0, 256, 4, 4, 7500.0), (0, 128, 4, 1, 7500.0), (1, 512, 4, 4, 900.0),
+    (1, 128, 4, 1, 900.0)])
+@pytest.mark.parametrize("n,rise", [(5, 7.75), (5, 6.9), (600, 7.75), (600, 6.9)])
+def test_prefill_weights_beyond_f16(gpu, ora, mode, D, bits, Hq, amp, n, rise):
+    """V scales of up to 483 (affine; valid below 511) and, past that, 950, and
+    norms / sqrt(D) of 450 and 900 (4-bit codebook), behind scores that rise
+    (base 2) after the first keys by less and by more than what moves the
+    reference maximum: weights p * scale of up to 1.1e5 where that is past
+    f16's 65504. There the pair is 65504 and a residual r <= 65504 rounded or
+    cut to 2^-10 of itself, hence good to 2^-11 of the weight, and the value
+    to 2^-11 of the longest row that it averages."""
     import torch
 
     prefix, Hkv = 700, 1
@@ -161,15 +164,54 @@ def test_prefill_weights_beyond_f16(gpu, ora, mode, D, bits, Hq, amp, n):
     oc.append(k[:prefix], v[:prefix])
     ks, vs = oc.dequant_kv()
     score = float(ks[-1, 0] @ (q[0, 0].astype(np.uint32) << 16).view(np.float32))
-    scale = float(np.float32(7.75 * np.log(2.0) / score))
+    scale = float(np.float32(rise * np.log(2.0) / score))
     held = oc.meta[:prefix, 1, 0].view(np.float16).astype(np.float64)
     held = np.abs(held[:, 0::2]) if mode == 0 else held / np.sqrt(D)
-    assert 65520 < 2.0 ** 7.75 * held.max() < 131008 and held.max() < 511
+    assert 450 <= 1.01 * held.max() and 2.0 ** 6.9 * held.max() < 131008
     cache = gpu.KVCache(gpu.make_desc(Hkv, D, bits, 0, cap, mode))
     cache.append(dev_bf16(k[:prefix]), dev_bf16(v[:prefix]))
     out = cache.prefill_step(dev_bf16(k[prefix:]), dev_bf16(v[prefix:]), dev_bf16(q), scale,
                              dtype=torch.float32)
     torch.cuda.synchronize()
     err = np.abs(out.cpu().numpy().astype(np.float64) - oc.prefill(k[prefix:], v[prefix:], q, scale))
-    bound = 2.0 ** -12 * np.sqrt((vs ** 2).sum(-1).max())
+    bound = 2.0 ** -11 * np.sqrt((vs ** 2).sum(-1).max())
     assert np.isfinite(err).all() and err.max() < bound, f"{err.max():.3e} of {bound:.3e}"
+
+
+@pytest.mark.parametrize("mode,D,bits,Hq", [
+    (0, 512, 8, 8), (0, 256, 4, 4), (0, 128, 8, 2), (1, 512, 4, 8), (1, 256, 3, 4), (1, 128, 2, 1),
+    (2, 512, 16, 8), (2, 256, 16, 4), (2, 128, 16, 1)])
+@pytest.mark.parametrize("window,bad", [(0, 707), (0, 723), (600, 113), (600, 701)])
+@pytest.mark.parametrize("n", [60, 2100])
+def test_prefill_hides_infinite_rows(gpu, ora, mode, D, bits, Hq, window, bad, n):
+    """A position whose V is infinite or past what a scale or norm holds: the queries before it and those whose window has left it are the
+    finite results of the other rows (n = 2100: on grids of their own, not
+    split over the keys); those that see it are not finite. bad: inside and at
+    the edge of the chunk's first key blocks, or in the prefix."""
+    import torch
+
+    prefix, Hkv = 693, 1
+    cap = prefix + n
+
+    def caches():
+        return (gpu.KVCache(gpu.make_desc(Hkv, D, bits, window, 0 if window else cap, mode)),
+                ora.OracleCache(Hkv, D, bits, window, 0 if window else cap, mode=mode))
+
+    cache, oc = caches()
+    k, v = kv_batch(n, cap, Hkv, D), kv_batch(n + 1, cap, Hkv, D)
+    vx = v.copy()
+    vx[bad, 0, 3] = 0xff80 if mode == 2 else 0x7f00  # -inf (else 1.7e38)
+    q = soft_q(n, n, Hq, D)
+    scale = 0.3 / np.sqrt(D)
+    cache.append(dev_bf16(k[:prefix]), dev_bf16(vx[:prefix]))
+    oc.append(k[:prefix], v[:prefix])
+    out = cache.prefill_step(dev_bf16(k[prefix:]), dev_bf16(vx[prefix:]), dev_bf16(q), scale,
+                             dtype=torch.float32).cpu().numpy().astype(np.float64)
+    pos = np.arange(prefix, cap)
+    sees = (pos >= bad) & ((pos < bad + window) if window else True)
+    rows = np.nonzero(~sees)[0]
+    rows = rows[(np.abs(pos[rows] - bad) < 80) | (np.abs(pos[rows] - bad - window) < 80)]
+    assert rows.size and sees.any() and not np.isfinite(out[sees]).all(axis=(1, 2)).any()
+    err = np.abs(out[rows] - oc.prefill(k[prefix:], v[prefix:], q, scale, rows=rows))
+    assert np.isfinite(out[~sees]).all()
+    assert err.max() < 2e-2 and err.mean() < 1.2e-4, f"{err.max():.2e} {err.mean():.2e}"
