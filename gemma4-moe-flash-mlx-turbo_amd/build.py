@@ -57,7 +57,7 @@ HIP_FLAGS = [
 
 # attention sources: contraction on, except where a pragma turns it off
 CONTRACT_SOURCES = {"fmkv_attention.hip", "fmkv_cb_attention.hip", "fmkv_plain_attention.hip",
-                    "fmkv_prefill.hip", "fmkv_prefill_short.hip"}
+                    "fmkv_prefill.hip"}
 # sources whose kernels take their first 14 argument dwords as scalars that
 # the dispatch preloads into SGPRs
 PRELOAD_SOURCES = {"fmkv_attention.hip"}

@@ -269,17 +269,11 @@ fmkv::Store pool_store(const fmkv_pool* p, const int32_t* table, int32_t stride)
 // memory for the partials: the unsplit launch needs none.
 hipError_t run_prefill(fmkv::PrefillArgs& pa, PrefillScratch& sc, int cus, int64_t max_steps,
                        hipStream_t s) {
-  if (fmkv::prefill_is_short(pa, max_steps)) return fmkv::launch_prefill_short(pa, s);
-  size_t bytes = 0;
-  int units = fmkv::prefill_units(pa, cus, max_steps, &bytes);
-  if (units > 0) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      units = 0;
-    }
-  }
-  if (units > 0 && bytes > sc.ws.bytes) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const bool captured = hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+  if (captured) (void)hipGetLastError();
+  size_t bytes = fmkv::prefill_plan(pa, cus, max_steps, !captured);
+  if (bytes > sc.ws.bytes) {
     float* ptr = nullptr;
     if (hipMalloc(&ptr, bytes) == hipSuccess) {
       sc.ws.release();  // (hipFree waits for the calls that use it)
@@ -287,16 +281,15 @@ hipError_t run_prefill(fmkv::PrefillArgs& pa, PrefillScratch& sc, int cus, int64
       sc.ws.bytes = bytes;
     } else {
       (void)hipGetLastError();
-      units = 0;
+      bytes = fmkv::prefill_plan(pa, cus, max_steps, false);
     }
   }
-  if (units > 0 && !sc.used && hipEventCreateWithFlags(&sc.used, hipEventDisableTiming) != hipSuccess) {
+  if (bytes > 0 && !sc.used && hipEventCreateWithFlags(&sc.used, hipEventDisableTiming) != hipSuccess) {
     (void)hipGetLastError();
     sc.used = nullptr;
-    units = 0;
+    bytes = fmkv::prefill_plan(pa, cus, max_steps, false);
   }
-  if (units == 0) return fmkv::launch_prefill_attention(pa, s);
-  pa.units = units;
+  if (bytes == 0) return fmkv::launch_prefill_attention(pa, s);
   pa.part_o = sc.ws.ptr;
   // (bytes = rows * (D + 2) floats)
   const int D = pa.new_st.layout.head_dim;

@@ -157,8 +157,11 @@ struct PrefillArgs {
   // partial rows go to part_o [units][n_kv_heads][tiles][64][D] and part_ml
   // [..][64][2] for a merge; 0: one work-group per (tile, KV head, sequence).
   int32_t units = 0;
+  int32_t min_split = 0;  // sequences of fewer steps of 32 keys stay one range
   float* part_o = nullptr;
   float* part_ml = nullptr;
+  // eight waves a work-group at head_dim 128 and 256 too, sharing its rows
+  bool share_rows = false;
 };
 
 struct ReadArgs {
@@ -242,14 +245,10 @@ hipError_t launch_sparse_gather(const AttnArgs& a, int n_seqs, hipStream_t s);
 // The split merge of every decode kernel: out = LSE merge of the partials.
 hipError_t launch_combine(const AttnArgs& a, int n_seqs, hipStream_t s);
 hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t s);
-// The same for short contexts (fmkv_prefill_short.hip), and whether a call in
-// which no sequence has more than max_steps steps of 32 keys is one.
-hipError_t launch_prefill_short(const PrefillArgs& a, hipStream_t s);
-bool prefill_is_short(const PrefillArgs& a, int64_t max_steps);
-// Units of a prefill call split over its keys (0: not worth it) on a GPU of
-// `cus` CUs, no sequence having more than max_steps steps of 32 keys, and the
-// bytes of its partials (part_o, then part_ml).
-int prefill_units(const PrefillArgs& a, int cus, int64_t max_steps, size_t* bytes);
+// How a prefill call runs on a GPU of `cus` CUs (share_rows, units and
+// min_split of a), no sequence having more than max_steps steps of 32 keys:
+// the bytes of its partials (part_o, then part_ml), 0 where it is not split.
+size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split);
 hipError_t launch_read_codes(const ReadArgs& a, hipStream_t s);
 hipError_t launch_fetch(const FetchArgs& a, hipStream_t s);
 

@@ -15,8 +15,10 @@
 // registers (no LDS staging), and is used for four 16-row tiles. (One pair of
 // waves per 16 rows, every pair decoding every block, took 7.78 ms for a
 // 2048-token chunk after 32768 positions, 16 q / 2 KV heads of 512 dims, 8
-// bits; this split takes 5.28 ms, and 0.148 against 0.227 ms for a 2048-token
-// chunk on a 1024-position ring, 16 / 8 heads of 256 dims, 4 bits.)
+// bits; this split takes 5.26 ms, and 0.150 against 0.227 ms for a 2048-token
+// chunk on a 1024-position ring, 16 / 8 heads of 256 dims, 4 bits.) Small grids
+// at head_dim 128 and 256 share the rows among eight waves, RW = 4 and 2 per 64
+// dims (prefill_plan).
 //
 // What bounds it: the issue of matrix and vector instructions together. A
 // 16x16x32 MFMA alone takes 8.7 ns of a SIMD, with four independent FMAs after
@@ -29,7 +31,7 @@
 //   QK^T  S_g^T[32 key x 64 row] = K_g . Q_g^T per wave: a partial score over
 //         its 64 dims, handed through LDS to the wave that sums the row's
 //         partials;
-//   softmax of 64 / (D / 64) rows per wave: sum, mask, running max, weights
+//   softmax of 64 / (number of waves) rows per wave: sum, mask, running max, weights
 //         P to LDS, and the factor by which every wave rescales its row
 //         accumulators when a row's reference max moved;
 //   PV    O_g^T[64 dim x 64 row] += V_g^T[64 dim x 32 key] . P^T[32 key x 64
@@ -74,7 +76,7 @@
 // sequence getting a number of ranges that follows its length
 // (prefill_unit), and a second kernel merges the ranges' partial rows. Four
 // 77-token chunks after 700 .. 8000 positions (16 q / 2 KV heads of 512 dims,
-// 3-bit codebook: 80 work-groups, the longest of 253 steps): 0.196 ms against
+// 3-bit codebook: 80 work-groups, the longest of 253 steps): 0.20 ms against
 // 0.575 unsplit.
 //
 // Keys come from two stores: positions below p_split from old_st (the ring
@@ -97,6 +99,7 @@ constexpr int kPfTiles = kPfRows / 16;
 constexpr int kPfKeys = 2 * kBlockTokens;  // keys per step
 constexpr int kPfQuads = kPfKeys / 4;      // groups of four keys of a step
 constexpr int kPfMinSteps = 4;             // steps of the shortest key range of a split call
+constexpr int kPfFewSteps = 32;            // a call of sequences shorter than this is short
 // How far (base 2) a score may exceed its row's reference maximum before the
 // row is rescaled. Weights stay below 2^7, and a weight times a V scale that an
 // affine cache's attention documents as valid (below 511) within f16. The
@@ -113,11 +116,15 @@ constexpr float kPfSlack = 7.0f;
 template <int BITS>
 constexpr float kPvScale = kCbExact<BITS> ? 32.0f : 1.0f;
 
-template <int D, int BITS, int MODE>
+// RW: ways that the 64 rows are shared among the waves (each dim group's
+// waves), 1 or as many as make eight waves
+template <int D, int BITS, int MODE, int RW>
 struct PfPlan {
   static constexpr BlockLayout L = make_layout(D, BITS, MODE);
   static constexpr int NG = D / 64;
-  static constexpr int NW = NG;  // waves: one per 64 dims
+  static constexpr int NW = NG * RW;  // waves: RW per 64 dims
+  static constexpr int PT = kPfTiles / RW;  // row tiles per wave
+  static_assert(RW == 1 || NW == 8, "eight waves where rows are shared");
   // The softmax stage: with 8 waves a wave sums 8 rows, lane l holding key
   // quad l >> 3 of row l & 7. With 4 (2) waves it sums one (two) whole row
   // tiles in the QK accumulators' own layout, so its own partial stays in
@@ -125,7 +132,7 @@ struct PfPlan {
   static constexpr bool kOwn = NW < 8;
   static constexpr int NRS = NW == 2 ? 2 : 1;  // row sets per lane
   static constexpr int NQ = kOwn ? 2 : 1;      // key quads per lane and row set
-  static constexpr int kSrc = kOwn ? NW - 1 : NW;  // partials of a tile in LDS
+  static constexpr int kSrc = kOwn ? NG - 1 : NG;  // partials of a tile in LDS
   static constexpr int kXs = kPfTiles * kSrc * 2 * 1024;  // one score buffer
   static constexpr int kPb = kPfQuads * kPfRows * 16;     // one weight buffer
   static constexpr int kPbOff = 2 * kXs;
@@ -183,13 +190,9 @@ __device__ inline uint32_t pack_bf16x2(float a, float b) {
 typedef const uint8_t __attribute__((address_space(1)))* gptr_t;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x2 u32x2_a4 __attribute__((aligned(4)));  // two words at a 4-byte boundary
-// The offset is opaque where it is used, or its extension to 64 bits leaves the
-// loop, and with it the form of the load that adds a 32-bit one to a scalar
-// base: 8 registers and 8 additions a step in a loop that is short of both.
 template <class T>
-__device__ inline T load_at(gptr_t p, uint32_t off) {
-  asm volatile("" : "+v"(off));
-  return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off);
+__device__ inline T load_at(gptr_t p, uint32_t off, int imm = 0) {
+  return *reinterpret_cast<const T __attribute__((address_space(1)))*>(p + off + imm);
 }
 
 // 2 N consecutive bf16 in one load a lane (aligned to one of them only).
@@ -240,6 +243,21 @@ __device__ inline int prefill_steps(const PrefillArgs& a, int64_t p0) {
   return (int)((keys > 0 ? keys : 0) / kPfKeys) + 2;
 }
 
+// Scalar loads of what every lane reads alike.
+typedef const int32_t __attribute__((address_space(4)))* cint_ptr;
+
+// The sums of lanes 0 .. l, in every lane l: DPP row shifts, then the last
+// lanes of rows broadcast over the rows after them.
+__device__ inline int scan_add(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+  return v;
+}
+
 // What unit u of the grid is: its sequence, the sequence's first unit and its
 // number of key ranges. The range length c is the smallest (to a sixteenth)
 // for which all sequences' ranges fit the units: the longest work-group, and
@@ -250,26 +268,30 @@ struct PrefillUnit {
   int seq, first, ranges;
 };
 __device__ inline PrefillUnit prefill_unit(const PrefillArgs& a, int u, int seq, int lane) {
+  // key ranges of a sequence of st steps, c steps each
+  auto count = [&](int st, int c) { return st < a.min_split ? 1 : (st + c - 1) / c; };
+  if (a.n_seqs == 1) {  // (the same, in scalar arithmetic)
+    const int st = prefill_steps(a, a.start_pos ? (int64_t)((cint_ptr)(uintptr_t)a.start_pos)[0] : a.p0);
+    int c = (st + a.units - 1) / a.units;
+    if (c < kPfMinSteps) c = kPfMinSteps;
+    const int n = count(st, c);
+    return PrefillUnit{u < n ? 0 : -1, 0, n};
+  }
   const int64_t p0 = lane < a.n_seqs ? (a.start_pos ? (int64_t)a.start_pos[lane] : a.p0) : 0;
-  const int st = lane < a.n_seqs ? prefill_steps(a, p0) : 0;
-  auto sum = [&](int v) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
-    return v;
-  };
-  int c = (sum(st) + a.units - 1) / a.units;
-  if (c < kPfMinSteps) c = kPfMinSteps;
-  int n = (st + c - 1) / c;
-  while (sum(n) > a.units) {  // ends: at c >= every st a sequence has one range, n_seqs <= units
-    c += 1 + c / 16;
-    n = (st + c - 1) / c;
+  const int st = prefill_steps(a, p0);
+  auto sum = [&](int v) { return (int)__builtin_amdgcn_readlane(scan_add(v), 63); };
+  int n = lane < a.n_seqs ? 1 : 0;
+  const uint64_t here = a.n_seqs < 64 ? (1ull << a.n_seqs) - 1 : ~0ull;
+  if (__ballot(st >= a.min_split) & here) {
+    int c = (sum(n ? st : 0) + a.units - 1) / a.units;
+    if (c < kPfMinSteps) c = kPfMinSteps;
+    n = n ? count(st, c) : 0;
+    while (sum(n) > a.units) {  // ends: at c >= every st a sequence has one range, n_seqs <= units
+      c += 1 + c / 16;
+      n = n ? count(st, c) : 0;
+    }
   }
-  int upto = n;  // units of sequences 0 .. lane
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) {
-    const int v = __shfl_up(upto, m);
-    if (lane >= m) upto += v;
-  }
+  const int upto = scan_add(n);  // units of sequences 0 .. lane
   PrefillUnit r;
   if (u >= 0) {
     const uint64_t past = __ballot(upto > u);
@@ -282,13 +304,13 @@ __device__ inline PrefillUnit prefill_unit(const PrefillArgs& a, int u, int seq,
   return r;
 }
 
-template <int D, int BITS, int MODE>
-__global__ __launch_bounds__(D)  // a wave per 64 dims
-__attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int D, int BITS, int MODE, int RW>
+__global__ __launch_bounds__(D * RW)  // RW waves per 64 dims
+__attribute__((amdgpu_waves_per_eu(RW == 4 ? 4 : 2, RW == 4 ? 4 : 2)))
 void prefill_attn_kernel(PrefillArgs a) {
-  using P = PfPlan<D, BITS, MODE>;
+  using P = PfPlan<D, BITS, MODE, RW>;
   constexpr BlockLayout L = P::L;
-  constexpr int NG = P::NG, NW = P::NW, E = D / 64, LPG = 64 / E;
+  constexpr int NG = P::NG, NW = P::NW, PT = P::PT, E = D / 64, LPG = 64 / E;
   constexpr int NRS = P::NRS, NQ = P::NQ, KW = P::KW, VW = P::VW;
   constexpr bool kOwn = P::kOwn;
   constexpr int QS = P::kQStride, RS = P::kRStride;
@@ -301,9 +323,14 @@ void prefill_attn_kernel(PrefillArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dg = RW > 1 ? wave % NG : wave, rt0 = RW > 1 ? wave / NG * PT : 0;  // dim group, first row tile
   const int j = lane >> 4, c = lane & 15;
   const int G = a.group;
   const int QP = kPfRows / G;  // query positions per work-group
+  const uint32_t g_inv = 65536u / (uint32_t)G + 1;
+  auto pos_of = [&](int r) __attribute__((always_inline)) {  // r / G for rows r < 64, G <= 64
+    return (int)((uint32_t)r * g_inv >> 16);
+  };
   const int kvh = blockIdx.y;
   int seq = blockIdx.z, range = 0, ranges = 1;
   if (a.units > 0) {
@@ -314,7 +341,6 @@ void prefill_attn_kernel(PrefillArgs a) {
   const int qi0 = blockIdx.x * QP;
   // paged: the sequence's start, through a scalar load (everything derived
   // from it stays in scalar registers)
-  typedef const int32_t __attribute__((address_space(4)))* cint_ptr;
   const int64_t p0 = a.start_pos ? (int64_t)((cint_ptr)(uintptr_t)a.start_pos)[seq] : a.p0;
   const int nq = a.n_q - qi0 < QP ? a.n_q - qi0 : QP;  // valid positions of the tile
 
@@ -373,7 +399,7 @@ void prefill_attn_kernel(PrefillArgs a) {
   const cint_ptr table =
       (cint_ptr)(uintptr_t)(a.new_st.block_table + (int64_t)seq * a.new_st.table_stride);
   auto blk_ptr = [&](int i) __attribute__((always_inline)) -> gptr_t {
-    i = i < nvb ? i : nvb - 1;
+    i = i < nvb ? i : nvb > 0 ? nvb - 1 : 0;
     if (i < n_old_i) {
       uint32_t phys = (uint32_t)(b_lo_i + i);
       if (nrb > 0) {
@@ -403,6 +429,128 @@ void prefill_attn_kernel(PrefillArgs a) {
     return vhi - vlo == kBlockTokens && vlo >= lo_max && vhi - 1 <= pA_r;
   };
 
+  // ---- this wave's loads: the codes (and scale / bias) of its 64 dims in
+  // the two blocks of a step ----
+  uint32_t kr[2][KW], vr[2][VW];
+  u32x4 km[2], vm[2];
+  const int kbit = (c * (D / 2) + (dg % (NG / 2)) * 64 + 8 * j) * CB;
+  const int vbit = (c * 16 + 4 * j) * CB;
+  const uint32_t ksh = kbit & 31, vsh = vbit & 31;
+  uint32_t k_off =
+      (int)L.k_codes +
+      (MODE == kAffine     ? (BITS == 8 ? dg * 1024 + lane * 16 : (dg >> 1) * 1024 + lane * 16 + (dg & 1) * 8)
+       : MODE == kCodebook ? (dg / (NG / 2)) * (D * CB) + (kbit >> 5) * 4
+                           : (c * D + dg * 64 + 8 * j) * 2);
+  uint32_t v_off =
+      (int)L.v_codes +
+      (MODE == kAffine     ? (BITS == 8 ? dg * 1024 + lane * 16 : (dg >> 1) * 1024 + lane * 16 + (dg & 1) * 8)
+       : MODE == kCodebook ? dg * (128 * CB) + (vbit >> 5) * 4
+                           : ((dg * 64 + c) * kBlockTokens + 4 * j) * 2);
+  uint32_t km_off = (int)L.k_meta + dg * 64 + j * 16;  // affine
+  uint32_t vm_off = (int)L.v_meta + dg * 64 + j * 16;
+  // Opaque in each step, or their extension to 64 bits leaves the loop, and
+  // with it the form of the loads that adds a 32-bit offset to a scalar base:
+  // 8 registers and 8 additions a step, in a loop that is short of both.
+  auto fresh_offsets = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(k_off), "+v"(v_off));
+    if constexpr (MODE == kAffine) asm volatile("" : "+v"(km_off), "+v"(vm_off));
+  };
+  auto load_k = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      if constexpr (MODE == kAffine) {
+        if constexpr (BITS == 8) {
+          const u32x4 w = load_at<u32x4>(bp[kt], k_off);
+#pragma unroll
+          for (int i = 0; i < 4; i++) kr[kt][i] = w[i];
+        } else {
+          const u32x2 w = load_at<u32x2>(bp[kt], k_off);
+          kr[kt][0] = w[0];
+          kr[kt][1] = w[1];
+        }
+        km[kt] = load_at<u32x4>(bp[kt], km_off);
+      } else if constexpr (MODE == kCodebook) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          if constexpr (CB == 3) {
+            const u32x2 w = load_at<u32x2_a4>(bp[kt], k_off, s * 4 * CB);
+            kr[kt][2 * s] = w[0];
+            kr[kt][2 * s + 1] = w[1];
+          } else {
+            kr[kt][s] = load_at<uint32_t>(bp[kt], k_off, s * 4 * CB);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const u32x4 w = load_at<u32x4>(bp[kt], k_off, s * 64);
+#pragma unroll
+          for (int i = 0; i < 4; i++) kr[kt][4 * s + i] = w[i];
+        }
+      }
+    }
+  };
+  auto load_v = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      if constexpr (MODE == kAffine) {
+        if constexpr (BITS == 8) {
+          const u32x4 w = load_at<u32x4>(bp[kt], v_off);
+#pragma unroll
+          for (int i = 0; i < 4; i++) vr[kt][i] = w[i];
+        } else {
+          const u32x2 w = load_at<u32x2>(bp[kt], v_off);
+          vr[kt][0] = w[0];
+          vr[kt][1] = w[1];
+        }
+        vm[kt] = load_at<u32x4>(bp[kt], vm_off);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+          if constexpr (MODE == kCodebook && CB != 3) {
+            vr[kt][n] = load_at<uint32_t>(bp[kt], v_off, n * 32 * CB);
+          } else {
+            const u32x2 w =
+                MODE == kCodebook ? (u32x2)load_at<u32x2_a4>(bp[kt], v_off, n * 32 * CB)
+                                  : load_at<u32x2>(bp[kt], v_off, n * 16 * kBlockTokens * 2);
+            vr[kt][2 * n] = w[0];
+            vr[kt][2 * n + 1] = w[1];
+          }
+        }
+      }
+    }
+  };
+  // codebook: the key norms of a step's softmax stage (K and V), the lane's
+  // own quads
+  u32x2 kn[NQ], vn[NQ];
+  const int quad0 = kOwn ? j : lane >> 3;  // the lane's first key quad (then quad0 + 4)
+  auto load_n = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
+    if constexpr (MODE == kCodebook) {
+#pragma unroll
+      for (int u = 0; u < NQ; u++) {
+        const gptr_t p = (kOwn ? u == 0 : quad0 < 4) ? bp[0] : bp[1];
+        kn[u] = load_at<u32x2>(p, (uint32_t)L.k_meta + 8 * (quad0 & 3));
+        vn[u] = load_at<u32x2>(p, (uint32_t)L.v_meta + 8 * (quad0 & 3));
+      }
+    }
+  };
+
+  // ---- the n steps from s_begin on ----
+  // (with several ranges, this one's share; possibly none)
+  const int per = ranges > 1 ? (nst + ranges - 1) / ranges : nst;
+  const int s_begin = range * per < nst ? range * per : nst;
+  // (a range that is left with none, and a sequence without keys: one step, all masked)
+  const int n = nst - s_begin < per ? (nst > s_begin ? nst - s_begin : 1) : per > 0 ? per : 1;
+  gptr_t cur[2], nxt[2], after[2];  // the blocks of steps i, i + 1, i + 2
+  bool f_cur = false, f_nxt = false, f_after = false;
+  // the blocks of step s_begin + i (past the end: of the last one)
+  auto blocks_of = [&](int i, gptr_t (&bp)[2], bool& f) __attribute__((always_inline)) {
+    if (i >= n) i = n - 1;
+    const int v = 2 * (s_begin + i);
+    bp[0] = blk_ptr(v);
+    bp[1] = blk_ptr(v + 1);
+    f = blk_full(v) && blk_full(v + 1);
+  };
   // ---- q_rot of the 64 rows: rows wave + NW k, high / residual halves
   // (plain: the raw bf16 rows) ----
   _Float16* const qhi = reinterpret_cast<_Float16*>(region);
@@ -411,26 +559,48 @@ void prefill_attn_kernel(PrefillArgs a) {
   if (tid == 0) not_finite = 0;
   const uint32_t sbits = lane_sign_bits<D>(a.sign_bits, lane);
   const float cs_lane = fwht_lane_sign(lane) * a.c;
-  // (eight rows' loads in flight together: one after the other, their latency
-  // made a 107-token chunk of head_dim 128, 32 rows a wave, twice as slow)
+  const int rows = nq * G;  // of the chunk
+  // Two rows at a time, the next two on their way meanwhile. (One at a time,
+  // the loads' latency made a 107-token chunk of head_dim 128, 32 rows a wave,
+  // twice as slow; eight unrolled take longer to fetch than to run.)
+  uint32_t raw[2][E / 2], ahead[2][E / 2];
+  auto load_q = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int rr = wave + NW * (k0 + k), r = rr < rows ? rr : rows - 1, rq = pos_of(r);
+      const int64_t row = ((int64_t)seq * a.n_q + qi0 + rq) * a.n_q_heads + (int64_t)kvh * G + (r - rq * G);
+      load_words<E / 2>(a.q + row * D + lane * E, ahead[k]);
+    }
+  };
+  auto zero_rows = [&](int k0) __attribute__((always_inline)) {  // the wave's from its k0th on
+    for (int r = wave + NW * k0; r < kPfRows; r += NW) {
+      const _Float16 z[E] = {};
+      store_halves<E>(reinterpret_cast<uint8_t*>(qhi + r * QS + lane * E), z);
+      if constexpr (MODE != kPlain)
+        store_halves<E>(reinterpret_cast<uint8_t*>(qlo + r * QS + lane * E), z);
+      if constexpr (MODE == kAffine)
+        if ((lane & (LPG - 1)) == 0) qsum[r * NG + ((lane * E) >> 6)] = 0.0f;
+    }
+  };
+  load_q(0);
+  // the first step's codes come in while the query rows are rotated (V's for
+  // the second time where they are used, but no more from memory)
+  blocks_of(0, cur, f_cur);
+  load_k(cur);
+  load_n(cur);
 #pragma unroll 1
-  for (int k0 = 0; k0 < kPfRows / NW; k0 += 8) {
-    uint32_t raw[8][E / 2];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int r = wave + NW * (k0 + k);
-      const int rq_ = r / G, rh_ = r - rq_ * G;
-      const int64_t qi = qi0 + (rq_ < nq ? rq_ : 0);
-      load_words<E / 2>(
-          a.q + (((int64_t)seq * a.n_q + qi) * a.n_q_heads + (int64_t)kvh * G + rh_) * D + lane * E,
-          raw[k]);
-      if (rq_ >= nq) {  // zero past the chunk
-#pragma unroll
-        for (int i = 0; i < E / 2; i++) raw[k][i] = 0;
-      }
+  for (int k0 = 0; k0 < kPfRows / NW; k0 += 2) {
+    if (wave + NW * k0 >= rows) {  // the rest is past the chunk: zeros
+      zero_rows(k0);
+      break;
     }
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int i = 0; i < E / 2; i++) raw[k][i] = ahead[k][i];
+    load_q(k0 + 2);  // (past the wave's last: a row of the chunk again)
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
       const int r = wave + NW * (k0 + k);
       if constexpr (MODE == kPlain) {
         uint32_t* dst = reinterpret_cast<uint32_t*>(qhi + r * QS + lane * E);
@@ -468,18 +638,18 @@ void prefill_attn_kernel(PrefillArgs a) {
   // holds 8 consecutive dims of row 16 rt + c at the K-code placement
   // (codebook and plain: slice s, dims 64 wave + 32 s + 8 j ..; plain B
   // operands are the bf16 bits)
-  half8_t bqh[kPfTiles][2], bql[kPfTiles][2];
-  float qs[kPfTiles];
+  half8_t bqh[PT][2], bql[PT][2];
+  float qs[PT];
 #pragma unroll
-  for (int rt = 0; rt < kPfTiles; rt++) {
-    const int row = rt * 16 + c;
+  for (int rt = 0; rt < PT; rt++) {
+    const int row = (rt0 + rt) * 16 + c;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-      const int d0 = wave * 64 + (MODE == kAffine && BITS == 8 ? j * 16 + s * 8 : s * 32 + j * 8);
+      const int d0 = dg * 64 + (MODE == kAffine && BITS == 8 ? j * 16 + s * 8 : s * 32 + j * 8);
       bqh[rt][s] = *reinterpret_cast<const half8_t*>(qhi + row * QS + d0);
       if constexpr (MODE != kPlain) bql[rt][s] = *reinterpret_cast<const half8_t*>(qlo + row * QS + d0);
     }
-    qs[rt] = MODE == kAffine ? qsum[row * NG + wave] : 0.0f;
+    qs[rt] = MODE == kAffine ? qsum[row * NG + dg] : 0.0f;
   }
   __syncthreads();  // the table is consumed: the region becomes the buffers
   uint8_t* const lut = region + P::kLutOff;
@@ -489,110 +659,11 @@ void prefill_attn_kernel(PrefillArgs a) {
     __syncthreads();
   }
 
-  // ---- this wave's loads: the codes (and scale / bias) of its 64 dims in
-  // the two blocks of a step ----
-  uint32_t kr[2][KW], vr[2][VW];
-  u32x4 km[2], vm[2];
-  const int kbit = (c * (D / 2) + (wave % (NG / 2)) * 64 + 8 * j) * CB;
-  const int vbit = (c * 16 + 4 * j) * CB;
-  const uint32_t ksh = kbit & 31, vsh = vbit & 31;
-  const uint32_t k_off =
-      (int)L.k_codes +
-      (MODE == kAffine     ? (BITS == 8 ? wave * 1024 + lane * 16 : (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8)
-       : MODE == kCodebook ? (wave / (NG / 2)) * (D * CB) + (kbit >> 5) * 4
-                           : (c * D + wave * 64 + 8 * j) * 2);
-  const uint32_t v_off =
-      (int)L.v_codes +
-      (MODE == kAffine     ? (BITS == 8 ? wave * 1024 + lane * 16 : (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8)
-       : MODE == kCodebook ? wave * (128 * CB) + (vbit >> 5) * 4
-                           : ((wave * 64 + c) * kBlockTokens + 4 * j) * 2);
-  const uint32_t km_off = (int)L.k_meta + wave * 64 + j * 16;  // affine
-  const uint32_t vm_off = (int)L.v_meta + wave * 64 + j * 16;
-  auto load_k = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      if constexpr (MODE == kAffine) {
-        if constexpr (BITS == 8) {
-          const u32x4 w = load_at<u32x4>(bp[kt], k_off);
-#pragma unroll
-          for (int i = 0; i < 4; i++) kr[kt][i] = w[i];
-        } else {
-          const u32x2 w = load_at<u32x2>(bp[kt], k_off);
-          kr[kt][0] = w[0];
-          kr[kt][1] = w[1];
-        }
-        km[kt] = load_at<u32x4>(bp[kt], km_off);
-      } else if constexpr (MODE == kCodebook) {
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-          if constexpr (CB == 3) {
-            const u32x2 w = load_at<u32x2_a4>(bp[kt], k_off + s * 4 * CB);
-            kr[kt][2 * s] = w[0];
-            kr[kt][2 * s + 1] = w[1];
-          } else {
-            kr[kt][s] = load_at<uint32_t>(bp[kt], k_off + s * 4 * CB);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-          const u32x4 w = load_at<u32x4>(bp[kt], k_off + s * 64);
-#pragma unroll
-          for (int i = 0; i < 4; i++) kr[kt][4 * s + i] = w[i];
-        }
-      }
-    }
-  };
-  auto load_v = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      if constexpr (MODE == kAffine) {
-        if constexpr (BITS == 8) {
-          const u32x4 w = load_at<u32x4>(bp[kt], v_off);
-#pragma unroll
-          for (int i = 0; i < 4; i++) vr[kt][i] = w[i];
-        } else {
-          const u32x2 w = load_at<u32x2>(bp[kt], v_off);
-          vr[kt][0] = w[0];
-          vr[kt][1] = w[1];
-        }
-        vm[kt] = load_at<u32x4>(bp[kt], vm_off);
-      } else {
-#pragma unroll
-        for (int n = 0; n < 4; n++) {
-          if constexpr (MODE == kCodebook && CB != 3) {
-            vr[kt][n] = load_at<uint32_t>(bp[kt], v_off + n * 32 * CB);
-          } else {
-            const u32x2 w =
-                MODE == kCodebook ? (u32x2)load_at<u32x2_a4>(bp[kt], v_off + n * 32 * CB)
-                                  : load_at<u32x2>(bp[kt], v_off + n * 16 * kBlockTokens * 2);
-            vr[kt][2 * n] = w[0];
-            vr[kt][2 * n + 1] = w[1];
-          }
-        }
-      }
-    }
-  };
-  // codebook: the key norms of a step's softmax stage (K and V), the lane's
-  // own quads
-  u32x2 kn[NQ], vn[NQ];
-  const int quad0 = kOwn ? j : lane >> 3;  // the lane's first key quad (then quad0 + 4)
-  auto load_n = [&](const gptr_t (&bp)[2]) __attribute__((always_inline)) {
-    if constexpr (MODE == kCodebook) {
-#pragma unroll
-      for (int u = 0; u < NQ; u++) {
-        const gptr_t p = (kOwn ? u == 0 : quad0 < 4) ? bp[0] : bp[1];
-        kn[u] = load_at<u32x2>(p, (uint32_t)L.k_meta + 8 * (quad0 & 3));
-        vn[u] = load_at<u32x2>(p, (uint32_t)L.v_meta + 8 * (quad0 & 3));
-      }
-    }
-  };
-
   // ---- the three stages ----
-  float4_t o[kPfTiles][4];  // [row tile][dim tile]: dims 16 ct + 4 j .., row 16 rt + c
-  float bacc[kPfTiles];
+  float4_t o[PT][4];  // [row tile][dim tile]: dims 16 ct + 4 j .., row 16 rt + c
+  float bacc[PT];
 #pragma unroll
-  for (int rt = 0; rt < kPfTiles; rt++) {
+  for (int rt = 0; rt < PT; rt++) {
     bacc[rt] = 0.0f;
 #pragma unroll
     for (int ct = 0; ct < 4; ct++) o[rt][ct] = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -604,9 +675,15 @@ void prefill_attn_kernel(PrefillArgs a) {
   // row of softmax row set u
   auto sm_row = [&](int u) __attribute__((always_inline)) { return kOwn ? (wave * NRS + u) * 16 + c : wave * 8 + (lane & 7); };
 
-  int p_row[NRS];  // the row's position
+  // a row's position (past the chunk: the last one, which sees nothing that
+  // no row does)
+  auto pos_at = [&](int r) __attribute__((always_inline)) {
+    const int rq = pos_of(r);
+    return pA_r + (rq < nq ? rq : nq - 1);
+  };
+  int p_row[NRS];
 #pragma unroll
-  for (int u = 0; u < NRS; u++) p_row[u] = pA_r + sm_row(u) / G;
+  for (int u = 0; u < NRS; u++) p_row[u] = pos_at(sm_row(u));
 
   float4_t* const xs = reinterpret_cast<float4_t*>(region);
   u32x4* const pb = reinterpret_cast<u32x4*>(region + P::kPbOff);
@@ -616,16 +693,16 @@ void prefill_attn_kernel(PrefillArgs a) {
     float4_t* const xb = xs + buf * (P::kXs / 16) + lane;
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      float4_t acc[kPfTiles];
+      float4_t acc[PT];
 #pragma unroll
-      for (int rt = 0; rt < kPfTiles; rt++) acc[rt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+      for (int rt = 0; rt < PT; rt++) acc[rt] = (float4_t){0.f, 0.f, 0.f, 0.f};
       if constexpr (MODE == kPlain) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
           const bf16x8_t ak = __builtin_bit_cast(
               bf16x8_t, (u32x4){kr[kt][4 * s], kr[kt][4 * s + 1], kr[kt][4 * s + 2], kr[kt][4 * s + 3]});
 #pragma unroll
-          for (int rt = 0; rt < kPfTiles; rt++)
+          for (int rt = 0; rt < PT; rt++)
             acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 ak, __builtin_bit_cast(bf16x8_t, bqh[rt][s]), acc[rt], 0, 0, 0);
         }
@@ -660,23 +737,23 @@ void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
         for (int s = 0; s < 2; s++)
 #pragma unroll
-          for (int rt = 0; rt < kPfTiles; rt++)
+          for (int rt = 0; rt < PT; rt++)
             acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bql[rt][s], acc[rt], 0, 0, 0);
         if constexpr (MODE == kCodebook && !kCbExact<CB>) {
 #pragma unroll
           for (int s = 0; s < 2; s++)
 #pragma unroll
-            for (int rt = 0; rt < kPfTiles; rt++)
+            for (int rt = 0; rt < PT; rt++)
               acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[s], bqh[rt][s], acc[rt], 0, 0, 0);
         }
 #pragma unroll
         for (int s = 0; s < 2; s++)
 #pragma unroll
-          for (int rt = 0; rt < kPfTiles; rt++)
+          for (int rt = 0; rt < PT; rt++)
             acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bqh[rt][s], acc[rt], 0, 0, 0);
       }
 #pragma unroll
-      for (int rt = 0; rt < kPfTiles; rt++) {
+      for (int rt = 0; rt < PT; rt++) {
         float4_t sv = acc[rt];
         if constexpr (MODE == kAffine) {
 #pragma unroll
@@ -690,15 +767,13 @@ void prefill_attn_kernel(PrefillArgs a) {
           else
             xb[((rt * P::kSrc + (wave < owner ? wave : wave - 1)) * 2 + kt) * 64] = sv;
         } else {
-          xb[((wave * 2 + kt) * kPfTiles + rt) * 64] = sv;
+          xb[((dg * 2 + kt) * kPfTiles + rt0 + rt) * 64] = sv;
         }
       }
     }
   };
 
-  // HIDE: as hide_not_finite
-  auto softmax = [&](int buf, int step, const float4_t (&mine)[NRS][2], bool full, auto hide) __attribute__((always_inline)) {
-    constexpr bool HIDE = decltype(hide)::value;
+  auto softmax = [&](int buf, int step, const float4_t (&mine)[NRS][2], bool full) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < NRS; u++) {
       const int row = sm_row(u);
@@ -758,7 +833,7 @@ void prefill_attn_kernel(PrefillArgs a) {
           for (int i = 0; i < 4; i++)
             if (!(kp + i >= vlo && kp + i < vhi)) {
               s[t][i] = -INFINITY;
-              if constexpr (HIDE && MODE == kCodebook) vscale[t][i] = 0.0f;
+              if constexpr (MODE == kCodebook) vscale[t][i] = 0.0f;  // (a norm may be infinite)
             }
         }
       }
@@ -787,23 +862,26 @@ void prefill_attn_kernel(PrefillArgs a) {
           // f16 high part and residual of P (affine) or of P' = p * norm /
           // sqrt D (codebook)
           half4_t h, r;
+          float rest[4];
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             float x = MODE == kCodebook ? p[i] * vscale[t][i] : p[i];
             // (one rounded product for both parts: fused into either conversion
             // it can round the high part to its other neighbour)
             asm("" : "+v"(x));
+            // (4 bits: norm / sqrt(D) has no bound. At most 65504 and a residual
+            // of as much, cut: infinite parts would meet as NaN. What is
+            // infinite or NaN before stays so, in the residual.)
             if constexpr (MODE == kCodebook && !kCbExact<CB>) {
-              // (4 bits: norm / sqrt(D) has no bound. At most 65504 and a
-              // residual of as much, cut: infinite parts would meet as NaN.
-              // What is infinite or NaN before stays so, in the residual.)
               h[i] = (_Float16)fminf(x, 65504.0f);
-              r[i] = pkrtz(x - (float)h[i], 0.0f)[0];
+              rest[i] = x - (float)h[i];
             } else {
               h[i] = (_Float16)x;
               r[i] = (_Float16)(x - (float)h[i]);
             }
           }
+          if constexpr (MODE == kCodebook && !kCbExact<CB>)
+            r = cat4(pkrtz(rest[0], rest[1]), pkrtz(rest[2], rest[3]));
           const uint2 hw = __builtin_bit_cast(uint2, h), rw = __builtin_bit_cast(uint2, r);
           w = (u32x4){hw.x, hw.y, rw.x, rw.y};
         } else {
@@ -820,10 +898,14 @@ void prefill_attn_kernel(PrefillArgs a) {
   };
 
   auto rescale = [&](int buf) __attribute__((always_inline)) {
-    const float4_t av = *reinterpret_cast<const float4_t*>(al + buf * kPfRows + c * 4);
-    if (__any(av[0] != 1.0f || av[1] != 1.0f || av[2] != 1.0f || av[3] != 1.0f)) {
+    typedef float av_t __attribute__((ext_vector_type(PT)));  // (one load)
+    const av_t av = *reinterpret_cast<const av_t*>(al + buf * kPfRows + c * 4 + rt0);
+    bool moved = false;
 #pragma unroll
-      for (int rt = 0; rt < kPfTiles; rt++) {
+    for (int rt = 0; rt < PT; rt++) moved = moved || av[rt] != 1.0f;
+    if (__any(moved)) {
+#pragma unroll
+      for (int rt = 0; rt < PT; rt++) {
 #pragma unroll
         for (int ct = 0; ct < 4; ct++) o[rt][ct] *= av[rt];
         bacc[rt] *= av[rt];
@@ -871,9 +953,9 @@ void prefill_attn_kernel(PrefillArgs a) {
       }
     }
 #pragma unroll
-    for (int rt = 0; rt < kPfTiles; rt++) {
-      const u32x4 w0 = pb[buf * (P::kPb / 16) + j * kPfRows + rt * 16 + c];
-      const u32x4 w1 = pb[buf * (P::kPb / 16) + (j + 4) * kPfRows + rt * 16 + c];
+    for (int rt = 0; rt < PT; rt++) {
+      const u32x4 w0 = pb[buf * (P::kPb / 16) + j * kPfRows + (rt0 + rt) * 16 + c];
+      const u32x4 w1 = pb[buf * (P::kPb / 16) + (j + 4) * kPfRows + (rt0 + rt) * 16 + c];
       half8_t bh, bl;
       if constexpr (MODE == kAffine) {
         // P' = p * v_scale in packed f16: the high part P_hi * s rounded, then
@@ -926,85 +1008,70 @@ void prefill_attn_kernel(PrefillArgs a) {
 
   // V values (affine: scales and biases) that are not finite, in a step whose
   // keys some rows do not see: a hidden key's weight 0 makes NaN of them. They
-  // become 0, and NaN the accumulators of the rows that do see them.
+  // become 0, and infinite (or NaN) the accumulators of the rows that do see
+  // them. (In arithmetic without compares: their masks would crowd the scalar
+  // registers of the whole kernel, and the loop ran up to 10% slower.)
   auto hide_not_finite = [&](int step) __attribute__((always_inline)) {
-    constexpr uint32_t kExp = MODE == kPlain ? 0x7f80u : 0x7c00u;
-    // all bits of the 16-bit values in w that are not finite
+    // 1 in each half of w that is not finite: its exponent is all ones
     auto bad_of = [&](uint32_t w) __attribute__((always_inline)) -> uint32_t {
-      return ((w & kExp) == kExp ? 0xffffu : 0u) |
-             ((w & (kExp << 16)) == (kExp << 16) ? 0xffff0000u : 0u);
+      constexpr uint32_t kExp = MODE == kPlain ? 0x7f807f80u : 0x7c007c00u;
+      constexpr uint32_t kOne = MODE == kPlain ? 0x00800080u : 0x04000400u;
+      return ((w & kExp) + kOne) >> 15 & 0x00010001u;
     };
-    // bit 4 kt + i: row 16 rt + c sees the lane's key 4 j + i of block kt
-    auto seen_of = [&](int rt) __attribute__((always_inline)) -> uint32_t {
-      const int p = pA_r + (rt * 16 + c) / G;
-      uint32_t m = 0;
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++) {
-        const int vi = 2 * step + kt, lo = lo_rel(p);
-        int vlo, vhi;
-        vb_range(vi, vlo, vhi);
-        vlo = vlo > lo ? vlo : lo;
-        vhi = vhi < p + 1 ? vhi : p + 1;
-        const int kp = (vi < n_old_i ? vi : vi + vb_shift) * kBlockTokens + 4 * j;
-#pragma unroll
-        for (int i = 0; i < 4; i++) m |= kp + i >= vlo && kp + i < vhi ? 1u << (4 * kt + i) : 0u;
-      }
-      return m;
+    // 1 for the keys 4 j + i of block kt that row 16 (rt0 + rt) + c sees, else 0
+    auto seen_of = [&](int rt, int kt, int i) __attribute__((always_inline)) -> uint32_t {
+      const int p = pos_at((rt0 + rt) * 16 + c), lo = lo_rel(p), vi = 2 * step + kt;
+      int vlo, vhi;
+      vb_range(vi, vlo, vhi);
+      vlo = vlo > lo ? vlo : lo;
+      vhi = vhi < p + 1 ? vhi : p + 1;
+      const int kp = (vi < n_old_i ? vi : vi + vb_shift) * kBlockTokens + 4 * j + i;
+      return ~(uint32_t)((kp - vlo) | (vhi - 1 - kp)) >> 31;
+    };
+    auto poison = [](float x, float n) __attribute__((always_inline)) -> float {  // n = 0: x
+      return fmaf(n * 0x1p127f, 0x1p127f, x);
     };
     if constexpr (MODE == kPlain) {
 #pragma unroll
-      for (int rt = 0; rt < kPfTiles; rt++) {
+      for (int rt = 0; rt < PT; rt++) {
         // how many of them a row sees, per dim: a product of ones
-        const uint32_t m = seen_of(rt);
         u32x4 seen;
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          seen[e] = (m >> (2 * e) & 1 ? 0x3f80u : 0u) | (m >> (2 * e) & 2 ? 0x3f800000u : 0u);
+          seen[e] = seen_of(rt, e >> 1, (e & 1) * 2) * 0x3f80u |
+                    seen_of(rt, e >> 1, (e & 1) * 2 + 1) * 0x3f800000u;
 #pragma unroll
         for (int ct = 0; ct < 4; ct++) {
           u32x4 bad;
 #pragma unroll
-          for (int e = 0; e < 4; e++) bad[e] = bad_of(vr[e >> 1][2 * ct + (e & 1)]) & 0x3f803f80u;
+          for (int e = 0; e < 4; e++) bad[e] = bad_of(vr[e >> 1][2 * ct + (e & 1)]) * 0x3f80u;
           const float4_t n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(bf16x8_t, bad), __builtin_bit_cast(bf16x8_t, seen),
               (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; i++) o[rt][ct][i] = n[i] > 0.0f ? NAN : o[rt][ct][i];
+          for (int i = 0; i < 4; i++) o[rt][ct][i] = poison(o[rt][ct][i], n[i]);
         }
       }
 #pragma unroll
       for (int w = 0; w < VW; w++) {
-        vr[0][w] &= ~bad_of(vr[0][w]);
-        vr[1][w] &= ~bad_of(vr[1][w]);
+        vr[0][w] &= ~(bad_of(vr[0][w]) * 0xffffu);
+        vr[1][w] &= ~(bad_of(vr[1][w]) * 0xffffu);
       }
     } else if constexpr (MODE == kAffine) {
-      uint32_t bad = 0;
 #pragma unroll
-      for (int b = 0; b < 8; b++) {
-        bad |= bad_of(vm[b >> 2][b & 3]) ? 1u << b : 0u;
-        vm[b >> 2][b & 3] = bad >> b & 1 ? 0u : vm[b >> 2][b & 3];
-      }
+      for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-      for (int rt = 0; rt < kPfTiles; rt++)  // (the lanes' sums join the row at the end)
-        bacc[rt] = bad & seen_of(rt) ? NAN : bacc[rt];
+        for (int i = 0; i < 4; i++) {
+          const uint32_t b = bad_of(vm[kt][i]), bad = (b | b >> 16) & 1u;
+          vm[kt][i] &= bad - 1u;
+#pragma unroll
+          for (int rt = 0; rt < PT; rt++)  // (the lanes' sums join the row at the end)
+            bacc[rt] = poison(bacc[rt], (float)(bad & seen_of(rt, kt, i)));
+        }
     }
   };
 
-  // ---- the pipeline over the n steps from s_begin on ----
-  // (with several ranges, this one's share; possibly none)
-  const int per = ranges > 1 ? (nst + ranges - 1) / ranges : nst;
-  const int s_begin = range * per < nst ? range * per : nst;
-  const int n = nst - s_begin < per ? nst - s_begin : per;
-  gptr_t cur[2], nxt[2], after[2];  // the blocks of steps i, i + 1, i + 2
-  bool f_cur = false, f_nxt = false, f_after = false;
-  // the blocks of step s_begin + i (past the end: of the last one)
-  auto blocks_of = [&](int i, gptr_t (&bp)[2], bool& f) __attribute__((always_inline)) {
-    if (i >= n) i = n - 1;
-    const int v = 2 * (s_begin + i);
-    bp[0] = blk_ptr(v);
-    bp[1] = blk_ptr(v + 1);
-    f = blk_full(v) && blk_full(v + 1);
-  };
+  // ---- the pipeline ----
   float4_t mine[NRS][2];
   auto keep_own = [&]() __attribute__((always_inline)) {
     if constexpr (kOwn) {
@@ -1018,43 +1085,39 @@ void prefill_attn_kernel(PrefillArgs a) {
     f_cur = f_nxt, f_nxt = f_after;
     blocks_of(i + 2, after, f_after);
   };
-  if (n > 0) {
-    blocks_of(0, cur, f_cur);
-    blocks_of(1, nxt, f_nxt);
-    blocks_of(2, after, f_after);
-    load_k(cur);
-    load_n(cur);
-    // the first interval's PV is of zero weights and codes
+  blocks_of(1, nxt, f_nxt);
+  blocks_of(2, after, f_after);
+  // the first interval's PV is of zero weights and codes
 #pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
+  for (int kt = 0; kt < 2; kt++) {
 #pragma unroll
-      for (int w = 0; w < VW; w++) vr[kt][w] = 0;
-      vm[kt] = (u32x4){0, 0, 0, 0};
-    }
-    for (int i = tid; i < P::kPb / 16; i += NW * 64) pb[P::kPb / 16 + i] = (u32x4){0, 0, 0, 0};
-    if (tid < kPfRows) al[kPfRows + tid] = 1.0f;
-    qk(0);
-    keep_own();
-    load_k(nxt);
-    lds_barrier();
-    // an interval between two barriers: QK of step i + 1 (past the end: of the
-    // last blocks, for nothing), softmax of step i, PV of step i - 1
-#pragma unroll 1
-    for (int i = 0; i < n; i++) {
-      rescale((i - 1) & 1);
-      qk((i + 1) & 1);
-      load_k(after);
-      softmax(i & 1, s_begin + i, mine, f_cur, std::false_type{});
-      keep_own();
-      load_n(nxt);
-      pv((i - 1) & 1, std::false_type{});
-      load_v(cur);
-      lds_barrier();
-      advance(i + 1);
-    }
-    rescale((n - 1) & 1);
-    pv((n - 1) & 1, std::false_type{});
+    for (int w = 0; w < VW; w++) vr[kt][w] = 0;
+    vm[kt] = (u32x4){0, 0, 0, 0};
   }
+  for (int i = tid; i < P::kPb / 16; i += NW * 64) pb[P::kPb / 16 + i] = (u32x4){0, 0, 0, 0};
+  if (tid < kPfRows) al[kPfRows + tid] = 1.0f;
+  qk(0);
+  keep_own();
+  load_k(nxt);
+  lds_barrier();
+  // an interval between two barriers: QK of step i + 1 (past the end: of the
+  // last blocks, for nothing), softmax of step i, PV of step i - 1
+#pragma unroll 1
+  for (int i = 0; i < n; i++) {
+    fresh_offsets();
+    rescale((i - 1) & 1);
+    qk((i + 1) & 1);
+    load_k(after);
+    softmax(i & 1, s_begin + i, mine, f_cur);
+    keep_own();
+    load_n(nxt);
+    pv((i - 1) & 1, std::false_type{});
+    load_v(cur);
+    lds_barrier();
+    advance(i + 1);
+  }
+  rescale((n - 1) & 1);
+  pv((n - 1) & 1, std::false_type{});
 
   // A sum that is not finite: some V value was not (or some score), and a row
   // that does not see it may have it all the same, as 0 * inf; or a V scale
@@ -1062,21 +1125,23 @@ void prefill_attn_kernel(PrefillArgs a) {
   // such values kept from those rows and such weights saturated. (Tested here
   // and not where V is read: a test in the steps with hidden keys alone cost
   // 2% of every call.)
-  bool bad = false;
+  // (Codebook caches: the norms are in the weights, 0 for a hidden key.)
+  if constexpr (MODE != kCodebook) {
+    float zero = 0.0f;
 #pragma unroll
-  for (int rt = 0; rt < kPfTiles; rt++) {
-    float s = MODE == kAffine ? bacc[rt] * 0.0f : 0.0f;
+    for (int rt = 0; rt < PT; rt++) {
+      if constexpr (MODE == kAffine) zero = fmaf(bacc[rt], 0.0f, zero);
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++)
+      for (int ct = 0; ct < 4; ct++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) s = fmaf(o[rt][ct][i], 0.0f, s);
-    bad = bad || s != 0.0f;
+        for (int i = 0; i < 4; i++) zero = fmaf(o[rt][ct][i], 0.0f, zero);
+    }
+    if (__any(zero != 0.0f)) not_finite = 1;
   }
-  if (__any(bad)) not_finite = 1;
   lds_barrier();  // the buffers are free
-  if (not_finite) {
+  if (MODE != kCodebook && not_finite) {
 #pragma unroll
-    for (int rt = 0; rt < kPfTiles; rt++) {
+    for (int rt = 0; rt < PT; rt++) {
       bacc[rt] = 0.0f;
 #pragma unroll
       for (int ct = 0; ct < 4; ct++) o[rt][ct] = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -1092,7 +1157,7 @@ void prefill_attn_kernel(PrefillArgs a) {
       qk(0);
       keep_own();
       lds_barrier();
-      softmax(0, s_begin + i, mine, f_cur, std::true_type{});
+      softmax(0, s_begin + i, mine, f_cur);
       lds_barrier();
       rescale(0);
       if (!f_cur) hide_not_finite(s_begin + i);
@@ -1111,11 +1176,11 @@ void prefill_attn_kernel(PrefillArgs a) {
   }
   float* const Rr = reinterpret_cast<float*>(region);
 #pragma unroll
-  for (int rt = 0; rt < kPfTiles; rt++) {
+  for (int rt = 0; rt < PT; rt++) {
     if constexpr (MODE == kAffine) bacc[rt] = xor32_sum(xor16_sum(bacc[rt]));
 #pragma unroll
     for (int ct = 0; ct < 4; ct++)
-      *reinterpret_cast<float4_t*>(&Rr[(rt * 16 + c) * RS + wave * 64 + ct * 16 + 4 * j]) =
+      *reinterpret_cast<float4_t*>(&Rr[((rt0 + rt) * 16 + c) * RS + dg * 64 + ct * 16 + 4 * j]) =
           MODE == kAffine     ? o[rt][ct] + bacc[rt]
           : MODE == kCodebook ? o[rt][ct] * (1.0f / kPvScale<CB>)
                               : o[rt][ct];
@@ -1136,7 +1201,7 @@ void prefill_attn_kernel(PrefillArgs a) {
     return;
   }
 #pragma unroll 1
-  for (int k0 = 0; k0 < kPfRows / NW; k0 += 4) {
+  for (int k0 = 0; k0 < kPfRows / NW && wave + NW * k0 < rows; k0 += 4) {
     float x[4][E];  // four rows at a time, past the chunk too (not stored)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -1152,7 +1217,7 @@ void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       const int r = wave + NW * (k0 + k);
-      const int rq_ = r / G, rh_ = r - rq_ * G;
+      const int rq_ = pos_of(r), rh_ = r - rq_ * G;
       if (rq_ >= nq) continue;
       const float l = lrow[r];
 #pragma unroll
@@ -1215,57 +1280,72 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int t
   }
 }
 
-template <int D, int BITS, int MODE>
-hipError_t launch_t(const PrefillArgs& a, hipStream_t s) {
+template <int D, int BITS, int MODE, int RW>
+hipError_t launch_rw(const PrefillArgs& a, hipStream_t s) {
   const int qp = kPfRows / a.group;
   const int tiles = (a.n_q + qp - 1) / qp, H = a.new_st.n_kv_heads;
   dim3 grid(tiles, H, a.units > 0 ? a.units : a.n_seqs);
-  hipLaunchKernelGGL((prefill_attn_kernel<D, BITS, MODE>), grid,
-                     dim3(PfPlan<D, BITS, MODE>::NW * 64), 0, s, a);
+  hipLaunchKernelGGL((prefill_attn_kernel<D, BITS, MODE, RW>), grid, dim3(D * RW), 0, s, a);
   if (a.units > 0) {
     dim3 mgrid(tiles * (kPfRows / kPfMergeRows), H, a.n_seqs);
     hipLaunchKernelGGL((prefill_merge_kernel<D, MODE != kPlain>), mgrid, dim3(256), 0, s, a, tiles);
   }
   return hipGetLastError();
 }
+template <int D, int BITS, int MODE>
+hipError_t launch_t(const PrefillArgs& a, hipStream_t s) {
+  if constexpr (D < 512)
+    if (a.share_rows) return launch_rw<D, BITS, MODE, 512 / D>(a, s);
+  return launch_rw<D, BITS, MODE, 1>(a, s);
+}
 
 }  // namespace
 
-// Short contexts go to fmkv_prefill_short.hip, up to where its time (first)
-// crosses this file's: 4-bit affine, 107 tokens after 50 (7 steps): 27 / 44 us
-// at head_dim 128, 34 / 39 at 256, 51 / 46 at 512; 4 x 300 after 200 (17
-// steps): 55 / 63, 117 / 96; 2 x 3 after 64 (4 steps): 18 / 33, 21 / 30, 32 /
-// 37; 20 after 400 (15 steps, split): 49 / 43, 59 / 42. Plain caches rotate
-// nothing: 2 x 3 after 64: 16 / 21, 18 / 19, 26 / 23; 107 after 50: 25 / 33,
-// 34 / 30.
-bool prefill_is_short(const PrefillArgs& a, int64_t max_steps) {
-  const int D = a.new_st.layout.head_dim;
-  if (a.new_st.layout.mode == kPlain) return max_steps <= (D == 128 ? 8 : D == 256 ? 4 : 0);
-  if (D == 128) {
-    // (few rows: the split of a longer context pays earlier)
-    const int64_t rows = (int64_t)a.n_seqs * a.n_q * a.n_q_heads;
-    return max_steps <= (rows >= 1024 ? 20 : 12);
-  }
-  return max_steps <= (D == 256 ? 8 : 4);
-}
-
-// The units of a split call (0: not split), and the bytes of its partials.
-// Worth it when one work-group per (tile, KV head, sequence) leaves at least
-// a whole round of CUs' places unused, so that the units all run at once, and
-// some sequence is long enough for two ranges. Work-groups per CU: the waves
-// that the registers of a SIMD hold, two, times four.
-int prefill_units(const PrefillArgs& a, int cus, int64_t max_steps, size_t* bytes) {
+// How a call runs. `total` counts its work-groups, one per (tile, KV head,
+// sequence); times are us per call with its append, 107 tokens after 50 written
+// 107@50.
+//
+// share_rows: the tile of a small grid at head_dim 128 and 256 goes to eight
+// waves instead of two and four. What a wave does once per row (rotations) then
+// takes a quarter or half of the time, and a step less, but each code is decoded
+// by four or two waves. Of short sequences that wins while every work-group has
+// a CU: 107@50, head_dim 128, affine 25 against 46, 256: 31 against 40; 4 x
+// 300@200 (160 work-groups), 128: 46 against 74; 800@100 (200), 256, 3-bit
+// codebook: 86 against 79, hence half the CUs there. Of long ones, which the key
+// ranges spread anyway, only a few rows win: 3@8000, 128: 47 against 52; 300@4000
+// of two sequences (80), 128: 92 against 86 (3-bit), 87 against 93 (affine);
+// 400@8000 (104), 256: 288 against 201. Head_dim 512 has eight waves in any case.
+//
+// places: work-groups that run at once. Registers allow two waves a SIMD (four
+// where a wave has one row tile): at head_dim 128 unshared that is four
+// work-groups a CU, of which three are counted, as the 3-bit codebook's 42 KB
+// of LDS allow no more.
+//
+// min_split: shorter sequences stay one range, and a call without longer ones
+// has no merge launch (about 4 us, also where it finds nothing to merge):
+// 107@50, 512: 46 one range, 51 two. A grid that fills part of the chip has
+// less to gain: 4 x 300@200, 128: 46 one range, 56 three each; but 512, whose
+// work-groups have a CU each: 400@0 (100, 14 steps): 62 two ranges, 66 one.
+size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) {
   const int D = a.new_st.layout.head_dim, qp = kPfRows / a.group;
   const int64_t wgs = (int64_t)((a.n_q + qp - 1) / qp) * a.new_st.n_kv_heads;  // per unit
-  const int64_t places = (int64_t)cus * (D == 512 ? 1 : D == 256 ? 2 : 3);
-  *bytes = 0;
-  if (a.n_seqs > 64 || max_steps < 2 * kPfMinSteps) return 0;
+  const int64_t total = wgs * a.n_seqs;
+  may_split = may_split && a.n_seqs <= 64;
+  const bool few = !may_split || max_steps < kPfFewSteps;
+  a.units = 0;
+  a.share_rows = D < 512 && total <= (!few ? cus / 4 : D == 128 ? cus : cus / 2);
+  const int64_t places =
+      (int64_t)cus * (D == 512 ? 1 : D == 256 ? (a.share_rows ? 1 : 2) : a.share_rows ? 2 : 3);
+  a.min_split = D == 512                            ? 8
+                : !a.share_rows && total <= cus ? 12
+                                                : (int)(12 + 16 * total / cus);
+  if (!may_split || max_steps < a.min_split) return 0;
   int64_t units = places / wgs;
   const int64_t most = a.n_seqs * ((max_steps + kPfMinSteps - 1) / kPfMinSteps);
   if (units > most) units = most;
-  if (units <= a.n_seqs) return 0;
-  *bytes = (size_t)(units * wgs * kPfRows) * (D + 2) * sizeof(float);
-  return (int)units;
+  if (2 * units < 3 * a.n_seqs) return 0;
+  a.units = (int)units;
+  return (size_t)(units * wgs * kPfRows) * (D + 2) * sizeof(float);
 }
 
 hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t s) {

@@ -215,3 +215,41 @@ def test_prefill_hides_infinite_rows(gpu, ora, mode, D, bits, Hq, window, bad, n
     err = np.abs(out[rows] - oc.prefill(k[prefix:], v[prefix:], q, scale, rows=rows))
     assert np.isfinite(out[~sees]).all()
     assert err.max() < 2e-2 and err.mean() < 1.2e-4, f"{err.max():.2e} {err.mean():.2e}"
+
+
+# every kernel instance: mode, bits, D
+INSTANCES = [(m, b, D) for m, bits in ((0, (4, 8)), (1, (2, 3, 4)), (2, (16,))) for b in bits for D in (128, 256, 512)]
+
+
+@pytest.mark.parametrize("mode,bits,D", INSTANCES)
+@pytest.mark.parametrize("prefix,n,wide", [(70, 3, 0), (70, 3, 3000), (1200, 3, 3000), (1, 97, 0), (1201, 97, 3000),
+                                           (1200, 800, 0), (30, 2100, 0)])
+def test_prefill_grids(gpu, ora, mode, bits, D, prefix, n, wide):
+    """Grids of 1, 13, 100 and 263 work-groups over short and long contexts,
+    on tables as wide as the sequence and far wider: rows shared by eight
+    waves or not, one key range or several, a merge that finds nothing to
+    merge. Every row finite, the first and last tiles' rows against the
+    oracle's exact attention. (A codebook row's reconstruction is not bounded
+    by its largest value: the path's own 2e-2 for the worst value there.)"""
+    import torch
+
+    Hkv, Hq, cap = 1, 8, prefix + n
+    oc = ora.OracleCache(Hkv, D, bits, 0, cap, mode=mode)
+    nb = (cap + 15) // 16
+    pool = gpu.PagedPool(gpu.make_desc(Hkv, D, bits, mode=mode), nb)
+    table = torch.zeros((1, max(nb, wide)), dtype=torch.int32, device="cuda")
+    table[0, :nb] = torch.arange(nb - 1, -1, -1, dtype=torch.int32, device="cuda")
+    k, v = kv_batch(prefix, cap, Hkv, D), kv_batch(prefix + 1, cap, Hkv, D)
+    q = soft_q(n, n, Hq, D)
+    scale = 0.3 / np.sqrt(D)
+    oc.append(k[:prefix], v[:prefix])
+    zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+    pool.append(dev_bf16(k[:prefix])[None], dev_bf16(v[:prefix])[None], table, zero)
+    args = [dev_bf16(x)[None] for x in (k[prefix:], v[prefix:], q)]
+    out = pool.prefill_step(args[0], args[1], table, zero + prefix, args[2], scale, dtype=torch.float32)
+    torch.cuda.synchronize()
+    out = out.cpu().numpy().astype(np.float64)[0]
+    assert np.isfinite(out).all()
+    rows = sorted({*range(min(n, 9)), *range(max(0, n - 9), n), n // 2})
+    err = np.abs(out[rows] - oc.prefill(k[prefix:], v[prefix:], q, scale, rows=rows))
+    assert err.max() < (2e-2 if mode == 1 else 4e-3) and err.mean() < 1.2e-4, f"{err.max():.2e} {err.mean():.2e}"
