@@ -191,18 +191,60 @@ struct Workspace {
   }
 };
 
-// The partials of a handle's split prefill calls. Calls on several streams
-// may be in flight (a prefill never needed a workspace of the handle before
-// its grid was split), so each use waits, on its stream, for the one before.
+constexpr int kMaxDevices = 64;
+
+// The partials of split prefill calls: one buffer per GPU for all its handles
+// (a call's partials live only while it runs, and a split grid fills the chip,
+// so two would not run side by side anyway). The first split call allocates it,
+// at the size that any call may need, and the last handle of the GPU frees it.
+// Calls on several streams and from several threads (of different handles) may
+// be in flight, so each use waits, on its stream, for the one before; the lock
+// keeps a use's wait, launches and record together.
 struct PrefillScratch {
-  Workspace ws;
+  std::mutex mu;
+  int handles = 0;
+  float* ptr = nullptr;
+  size_t bytes = 0;
   hipEvent_t used = nullptr;
-  void release() {
-    ws.release();
-    if (used) (void)hipEventDestroy(used);
-    used = nullptr;
+
+  // The buffer is there (false: no memory for it). Not a reason for a capture
+  // on another stream or thread to fail: allocating is allowed in this
+  // thread's relaxed mode.
+  bool ready(int cus) {
+    if (ptr) return true;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    bytes = fmkv::prefill_scratch_bytes(cus);
+    if (hipMalloc(&ptr, bytes) != hipSuccess) ptr = nullptr;
+    if (ptr && hipEventCreateWithFlags(&used, hipEventDisableTiming) != hipSuccess) {
+      (void)hipFree(ptr);
+      ptr = nullptr;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ptr) (void)hipGetLastError();
+    return ptr != nullptr;
   }
 };
+PrefillScratch g_prefill_scratch[kMaxDevices];
+
+// A handle's part in its GPU's scratch, from its creation to its end.
+PrefillScratch* prefill_scratch_join() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  PrefillScratch* sc = &g_prefill_scratch[dev];
+  std::lock_guard<std::mutex> lock(sc->mu);
+  sc->handles++;
+  return sc;
+}
+void prefill_scratch_leave(PrefillScratch* sc) {
+  if (!sc) return;
+  std::lock_guard<std::mutex> lock(sc->mu);
+  if (--sc->handles > 0 || !sc->ptr) return;
+  (void)hipFree(sc->ptr);  // (waits for the calls that use it)
+  (void)hipEventDestroy(sc->used);
+  sc->ptr = nullptr;
+  sc->used = nullptr;
+}
 
 }  // namespace
 
@@ -218,7 +260,7 @@ struct fmkv_cache {
   int64_t vis_begin;
   Workspace ws;
   Workspace stage;  // prefill on a ring: the chunk's quantized rows
-  PrefillScratch split;
+  PrefillScratch* split = nullptr;
   int cus;
 };
 
@@ -231,7 +273,7 @@ struct fmkv_pool {
   uint32_t sign_bits[16];
   float c, sqrt_d;
   Workspace ws;
-  PrefillScratch split;
+  PrefillScratch* split = nullptr;
   int cus;
 };
 
@@ -264,41 +306,30 @@ fmkv::Store pool_store(const fmkv_pool* p, const int32_t* table, int32_t stride)
 }
 
 // The prefill attention, split over its keys when the grid alone would leave
-// CUs idle. Not under stream capture (the scratch may have to grow, and a
-// replay is not ordered with other uses of it) and not when there is no
-// memory for the partials: the unsplit launch needs none.
-hipError_t run_prefill(fmkv::PrefillArgs& pa, PrefillScratch& sc, int cus, int64_t max_steps,
+// CUs idle. Not under stream capture (a replay would not be ordered with other
+// uses of the partials) and not when there is no memory for the partials: the
+// unsplit launch needs none.
+hipError_t run_prefill(fmkv::PrefillArgs& pa, PrefillScratch* sc, int cus, int64_t max_steps,
                        hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   const bool captured = hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
   if (captured) (void)hipGetLastError();
-  size_t bytes = fmkv::prefill_plan(pa, cus, max_steps, !captured);
-  if (bytes > sc.ws.bytes) {
-    float* ptr = nullptr;
-    if (hipMalloc(&ptr, bytes) == hipSuccess) {
-      sc.ws.release();  // (hipFree waits for the calls that use it)
-      sc.ws.ptr = ptr;
-      sc.ws.bytes = bytes;
-    } else {
-      (void)hipGetLastError();
-      bytes = fmkv::prefill_plan(pa, cus, max_steps, false);
-    }
-  }
-  if (bytes > 0 && !sc.used && hipEventCreateWithFlags(&sc.used, hipEventDisableTiming) != hipSuccess) {
-    (void)hipGetLastError();
-    sc.used = nullptr;
-    bytes = fmkv::prefill_plan(pa, cus, max_steps, false);
-  }
+  const size_t bytes = fmkv::prefill_plan(pa, cus, max_steps, sc && !captured);
   if (bytes == 0) return fmkv::launch_prefill_attention(pa, s);
-  pa.part_o = sc.ws.ptr;
+  std::lock_guard<std::mutex> lock(sc->mu);
+  if (!sc->ready(cus) || bytes > sc->bytes) {
+    (void)fmkv::prefill_plan(pa, cus, max_steps, false);
+    return fmkv::launch_prefill_attention(pa, s);
+  }
+  pa.part_o = sc->ptr;
   // (bytes = rows * (D + 2) floats)
   const int D = pa.new_st.layout.head_dim;
-  pa.part_ml = sc.ws.ptr + bytes / sizeof(float) / (D + 2) * D;
-  hipError_t e = hipStreamWaitEvent(s, sc.used, 0);
+  pa.part_ml = sc->ptr + bytes / sizeof(float) / (D + 2) * D;
+  hipError_t e = hipStreamWaitEvent(s, sc->used, 0);
   if (e != hipSuccess) return e;
   e = fmkv::launch_prefill_attention(pa, s);
   if (e != hipSuccess) return e;
-  return hipEventRecord(sc.used, s);
+  return hipEventRecord(sc->used, s);
 }
 
 int64_t visible_begin(const fmkv_cache* c) {
@@ -672,7 +703,6 @@ static __device__ __align__(256) uint8_t scratch[FMKV_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_dev[kMaxDevices] = {};
 
@@ -748,6 +778,7 @@ int fmkv_cache_create(const fmkv_cache_desc* desc, fmkv_cache** out) {
   }
   sign_bits_of(*desc, c->sign_bits);
   c->cus = device_cus();
+  c->split = prefill_scratch_join();
   // set-up of the no-allocation decode step's scratch on this device (once
   // per device; later creations find the address recorded)
   ExtWorkspace ext;
@@ -766,7 +797,7 @@ int fmkv_cache_destroy(fmkv_cache* c) {
   if (c->d_signs) (void)hipFree(c->d_signs);
   c->ws.release();
   c->stage.release();
-  c->split.release();
+  prefill_scratch_leave(c->split);
   delete c;
   return FMKV_OK;
 }
@@ -1081,6 +1112,7 @@ int fmkv_pool_create(const fmkv_cache_desc* desc, int64_t n_blocks, fmkv_pool** 
   }
   sign_bits_of(*desc, p->sign_bits);
   p->cus = device_cus();
+  p->split = prefill_scratch_join();
   *out = p;
   return FMKV_OK;
 }
@@ -1090,7 +1122,7 @@ int fmkv_pool_destroy(fmkv_pool* p) {
   if (p->arena) (void)hipFree(p->arena);
   if (p->d_signs) (void)hipFree(p->d_signs);
   p->ws.release();
-  p->split.release();
+  prefill_scratch_leave(p->split);
   delete p;
   return FMKV_OK;
 }

@@ -249,6 +249,8 @@ hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t s);
 // min_split of a), no sequence having more than max_steps steps of 32 keys:
 // the bytes of its partials (part_o, then part_ml), 0 where it is not split.
 size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split);
+// The most that prefill_plan returns on such a GPU.
+size_t prefill_scratch_bytes(int cus);
 hipError_t launch_read_codes(const ReadArgs& a, hipStream_t s);
 hipError_t launch_fetch(const FetchArgs& a, hipStream_t s);
 

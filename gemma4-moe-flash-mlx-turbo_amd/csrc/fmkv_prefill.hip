@@ -1301,6 +1301,24 @@ hipError_t launch_t(const PrefillArgs& a, hipStream_t s) {
 
 }  // namespace
 
+namespace {
+int64_t prefill_places(int D, bool share_rows, int cus) {
+  return (int64_t)cus * (D == 512 ? 1 : D == 256 ? (share_rows ? 1 : 2) : share_rows ? 2 : 3);
+}
+size_t prefill_part_bytes(int64_t work_groups, int D) {
+  return (size_t)(work_groups * kPfRows) * (D + 2) * sizeof(float);
+}
+}  // namespace
+
+size_t prefill_scratch_bytes(int cus) {
+  size_t most = 0;
+  for (int D : {128, 256, 512}) {
+    const size_t b = prefill_part_bytes(prefill_places(D, false, cus), D);
+    if (b > most) most = b;
+  }
+  return most;
+}
+
 // How a call runs. `total` counts its work-groups, one per (tile, KV head,
 // sequence); times are us per call with its append, 107 tokens after 50 written
 // 107@50.
@@ -1334,8 +1352,7 @@ size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) 
   const bool few = !may_split || max_steps < kPfFewSteps;
   a.units = 0;
   a.share_rows = D < 512 && total <= (!few ? cus / 4 : D == 128 ? cus : cus / 2);
-  const int64_t places =
-      (int64_t)cus * (D == 512 ? 1 : D == 256 ? (a.share_rows ? 1 : 2) : a.share_rows ? 2 : 3);
+  const int64_t places = prefill_places(D, a.share_rows, cus);
   a.min_split = D == 512                            ? 8
                 : !a.share_rows && total <= cus ? 12
                                                 : (int)(12 + 16 * total / cus);
@@ -1345,7 +1362,7 @@ size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) 
   if (units > most) units = most;
   if (2 * units < 3 * a.n_seqs) return 0;
   a.units = (int)units;
-  return (size_t)(units * wgs * kPfRows) * (D + 2) * sizeof(float);
+  return prefill_part_bytes(units * wgs, D);
 }
 
 hipError_t launch_prefill_attention(const PrefillArgs& a, hipStream_t s) {

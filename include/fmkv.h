@@ -16,7 +16,8 @@
  *    or f32 (FMKV_DTYPE_*). q head h reads KV head h / (n_q_heads/n_kv_heads).
  *  - `stream` is a hipStream_t (NULL = default stream). Every call is
  *    stream-ordered and asynchronous unless stated; nothing synchronises.
- *  - A handle is used by one host thread at a time (no internal locks).
+ *  - A handle is used by one host thread at a time (no lock of its own);
+ *    different handles by different threads.
  *  - Descriptor validation runs before any HIP call, so invalid input is
  *    reported on machines without a GPU too.
  *  - Magnitude bound of the affine attention read: the softmax weight times
@@ -213,7 +214,17 @@ int fmkv_decode_step_noalloc(fmkv_cache* cache, const void* k_bf16, const void* 
  * every query sees its whole window. out: [n_tokens][n_q_heads][D] in
  * out_dtype. Every cache mode (codebook caches are read as stored, plain
  * caches as their bf16 rows); at most 8 query heads per KV head;
- * n_tokens >= 1. Nothing is launched or changed when validation fails. */
+ * n_tokens >= 1. Nothing is launched or changed when validation fails.
+ *
+ * A call of few rows over a long context is split over its keys. The split
+ * calls of a GPU's handles share one buffer of partial rows (at most
+ * 132 KiB per CU: 33 MiB on 256), which the first of them allocates and the
+ * GPU's last handle to be destroyed frees; on several streams they wait for
+ * one another's use of it, on the device. Under stream capture, or without
+ * memory for the buffer, a call is not split. The split changes the order of
+ * the f32 sums, so the last bits of an output depend on whether the call is
+ * captured and, in a batch, on the other sequences' lengths and the block
+ * table's width; the same call on the same data gives the same bits. */
 int fmkv_prefill_step(fmkv_cache* cache, const void* k_bf16, const void* v_bf16, int64_t n_tokens,
                       const void* q_bf16, int32_t n_q_heads, float scale, void* out,
                       int32_t out_dtype, void* stream);
@@ -301,7 +312,8 @@ int fmkv_paged_decode_step_projected(fmkv_pool* pool, const void* k_proj_bf16,
  * :84-104 with L > 1, mask of create_attention_mask, src/model/mod.rs
  * :682-704) -- fmkv_prefill_step for a batch of requests. q: bf16
  * [n_seqs][n_new][n_q_heads][head_dim]; out: the same shape in out_dtype.
- * Every cache mode; at most 8 query heads per KV head. */
+ * Every cache mode; at most 8 query heads per KV head. The key split, its
+ * buffer and the order of sums: see fmkv_prefill_step. */
 int fmkv_paged_prefill_step(fmkv_pool* pool, const void* k_bf16, const void* v_bf16,
                             const int32_t* block_tables, int32_t max_blocks,
                             const int32_t* start_pos, int32_t n_seqs, int32_t n_new,
