@@ -1132,7 +1132,17 @@ int fmkv_paged_prefill_step(fmkv_pool* p, const void* k, const void* v,
                             const int32_t* start_pos, int32_t n_seqs, int32_t n_new,
                             const void* q, int32_t n_q_heads, float scale, void* out,
                             int32_t out_dtype, void* stream) {
+  return fmkv_paged_prefill_step_bounded(p, k, v, block_tables, max_blocks, start_pos, n_seqs,
+                                         n_new, 0, q, n_q_heads, scale, out, out_dtype, stream);
+}
+
+int fmkv_paged_prefill_step_bounded(fmkv_pool* p, const void* k, const void* v,
+                                    const int32_t* block_tables, int32_t max_blocks,
+                                    const int32_t* start_pos, int32_t n_seqs, int32_t n_new,
+                                    int32_t max_seq_len, const void* q, int32_t n_q_heads,
+                                    float scale, void* out, int32_t out_dtype, void* stream) {
   if (!p) return fail(FMKV_ERR_INVALID_ARG, "pool is null");
+  if (max_seq_len < 0) return fail(FMKV_ERR_INVALID_ARG, "max_seq_len must be >= 0 (0: unknown)");
   if (n_seqs < 1 || n_new < 1)
     return fail(FMKV_ERR_INVALID_ARG, "a prefill step needs n_seqs >= 1 and n_new >= 1");
   int rc = check_attn_args(p->desc, q, n_q_heads, 0.0f, out, out_dtype);
@@ -1169,8 +1179,10 @@ int fmkv_paged_prefill_step(fmkv_pool* p, const void* k, const void* v,
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e = fmkv::launch_append(ap, n_seqs, tasks, s);
   if (e != hipSuccess) return hip_fail(e, "paged append launch");
-  // (starts are on the device: the table's width bounds the lengths)
-  e = run_prefill(pa, p->split, p->cus, (int64_t)max_blocks / 2 + 2, s);
+  // (starts are on the device: the caller or the table's width bounds the lengths)
+  int64_t blocks = ((int64_t)max_seq_len + fmkv::kBlockTokens - 1) / fmkv::kBlockTokens;
+  if (blocks == 0 || blocks > max_blocks) blocks = max_blocks;
+  e = run_prefill(pa, p->split, p->cus, blocks / 2 + 2, s);
   if (e != hipSuccess) return hip_fail(e, "prefill attention launch");
   return FMKV_OK;
 }

@@ -1343,7 +1343,9 @@ size_t prefill_scratch_bytes(int cus) {
 // has no merge launch (about 4 us, also where it finds nothing to merge):
 // 107@50, 512: 46 one range, 51 two. A grid that fills part of the chip has
 // less to gain: 4 x 300@200, 128: 46 one range, 56 three each; but 512, whose
-// work-groups have a CU each: 400@0 (100, 14 steps): 62 two ranges, 66 one.
+// work-groups have a CU each: 400@0 (100, 14 steps): 62 two ranges, 66 one; and
+// where the bound is long, the merge launch being there anyway (a wide table's
+// 2 x 150@100, 256: 47 two ranges, 53 one).
 size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) {
   const int D = a.new_st.layout.head_dim, qp = kPfRows / a.group;
   const int64_t wgs = (int64_t)((a.n_q + qp - 1) / qp) * a.new_st.n_kv_heads;  // per unit
@@ -1353,9 +1355,7 @@ size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) 
   a.units = 0;
   a.share_rows = D < 512 && total <= (!few ? cus / 4 : D == 128 ? cus : cus / 2);
   const int64_t places = prefill_places(D, a.share_rows, cus);
-  a.min_split = D == 512                            ? 8
-                : !a.share_rows && total <= cus ? 12
-                                                : (int)(12 + 16 * total / cus);
+  a.min_split = D == 512 || (total <= cus && !(few && a.share_rows)) ? 8 : (int)(12 + 16 * total / cus);
   if (!may_split || max_steps < a.min_split) return 0;
   int64_t units = places / wgs;
   const int64_t most = a.n_seqs * ((max_steps + kPfMinSteps - 1) / kPfMinSteps);

@@ -50,7 +50,8 @@ EXPORTED = (
     "fmkv_cache_decode_splits",
     "fmkv_profile_enable", "fmkv_profile_collect", "fmkv_profile_collect_each",
     "fmkv_decode_step", "fmkv_paged_decode_step",
-    "fmkv_prefill_step", "fmkv_paged_prefill_step", "fmkv_decode_step_noalloc",
+    "fmkv_prefill_step", "fmkv_paged_prefill_step", "fmkv_paged_prefill_step_bounded",
+    "fmkv_decode_step_noalloc",
     "fmkv_decode_step_projected", "fmkv_paged_decode_step_projected",
 )
 
@@ -158,6 +159,8 @@ def load_library(path: str | os.PathLike | None = None) -> ctypes.CDLL:
         "fmkv_prefill_step": ([vp, vp, vp, i64, vp, i32, ctypes.c_float, vp, i32, vp], ctypes.c_int),
         "fmkv_paged_prefill_step": ([vp, vp, vp, vp, i32, vp, i32, i32, vp, i32, ctypes.c_float, vp,
                                      i32, vp], ctypes.c_int),
+        "fmkv_paged_prefill_step_bounded": ([vp, vp, vp, vp, i32, vp, i32, i32, i32, vp, i32,
+                                             ctypes.c_float, vp, i32, vp], ctypes.c_int),
         "fmkv_paged_decode_step": ([vp, vp, vp, vp, i32, vp, vp, i32, i32, i32, vp, i32,
                                     ctypes.c_float, ctypes.c_float, vp, i32, vp], ctypes.c_int),
         "fmkv_decode_step_projected": ([vp, vp, vp, i64, P(KvPrologue), vp, i32, ctypes.c_float,
@@ -545,18 +548,20 @@ class PagedPool:
             _ptr(start_pos), n_seqs, n_new, ctypes.byref(prologue), _stream(stream)))
 
     def prefill_step(self, keys, values, block_tables, start_pos, q, scale: float = 1.0,
-                     out=None, dtype=torch.bfloat16, stream=None):
+                     out=None, dtype=torch.bfloat16, stream=None, max_seq_len: int = 0):
         """append(keys, values, ...) at start_pos, then each sequence's causal
         attention of its n_new queries. keys/values bf16 [n_seqs, n_new,
-        n_kv_heads, D]; q bf16 [n_seqs, n_new, n_q_heads, D]."""
+        n_kv_heads, D]; q bf16 [n_seqs, n_new, n_q_heads, D]. max_seq_len: the
+        longest sequence's length after the call, where the host knows it (for
+        speed only, on tables wider than that; 0: the table's width)."""
         if q.dim() != 4 or q.shape[:2] != keys.shape[:2]:
             raise ValueError("q must be bf16 [n_seqs, n_new, n_q_heads, head_dim]")
         if out is None:
             out = torch.empty(q.shape, dtype=dtype, device=q.device)
-        _check(self._lib.fmkv_paged_prefill_step(
+        _check(self._lib.fmkv_paged_prefill_step_bounded(
             self._h, _ptr(keys), _ptr(values), _ptr(block_tables), block_tables.shape[1],
-            _ptr(start_pos), keys.shape[0], keys.shape[1], _ptr(q), q.shape[2], scale, _ptr(out),
-            _dtype_code(out.dtype), _stream(stream)))
+            _ptr(start_pos), keys.shape[0], keys.shape[1], max_seq_len, _ptr(q), q.shape[2], scale,
+            _ptr(out), _dtype_code(out.dtype), _stream(stream)))
         return out
 
     def attention(self, q, block_tables, seq_lens, max_seq_len: int, scale: float = 1.0,

@@ -218,7 +218,7 @@ int fmkv_decode_step_noalloc(fmkv_cache* cache, const void* k_bf16, const void* 
  *
  * A call of few rows over a long context is split over its keys. The split
  * calls of a GPU's handles share one buffer of partial rows (at most
- * 132 KiB per CU: 33 MiB on 256), which the first of them allocates and the
+ * 129 KiB per CU: 32.3 MiB on 256), which the first of them allocates and the
  * GPU's last handle to be destroyed frees; on several streams they wait for
  * one another's use of it, on the device. Under stream capture, or without
  * memory for the buffer, a call is not split. The split changes the order of
@@ -313,12 +313,27 @@ int fmkv_paged_decode_step_projected(fmkv_pool* pool, const void* k_proj_bf16,
  * :682-704) -- fmkv_prefill_step for a batch of requests. q: bf16
  * [n_seqs][n_new][n_q_heads][head_dim]; out: the same shape in out_dtype.
  * Every cache mode; at most 8 query heads per KV head. The key split, its
- * buffer and the order of sums: see fmkv_prefill_step. */
+ * buffer and the order of sums: see fmkv_prefill_step. How the work is laid
+ * out follows the longest length that the table's width allows;
+ * fmkv_paged_prefill_step_bounded takes it from the caller. */
 int fmkv_paged_prefill_step(fmkv_pool* pool, const void* k_bf16, const void* v_bf16,
                             const int32_t* block_tables, int32_t max_blocks,
                             const int32_t* start_pos, int32_t n_seqs, int32_t n_new,
                             const void* q_bf16, int32_t n_q_heads, float scale, void* out,
                             int32_t out_dtype, void* stream);
+
+/* fmkv_paged_prefill_step with the length of the longest sequence after the
+ * call (its start_pos + n_new), where the host knows it, as
+ * fmkv_paged_decode_step takes it; 0: as the table's width allows. Only speed
+ * depends on it, and a wrong one gives right results: on tables much wider
+ * than their sequences it saves short calls a launch (4 us) and picks the
+ * better work-groups (4 x 100 tokens after 30, 16 q / 8 KV heads of 256 dims:
+ * 45 -> 32 us). */
+int fmkv_paged_prefill_step_bounded(fmkv_pool* pool, const void* k_bf16, const void* v_bf16,
+                                    const int32_t* block_tables, int32_t max_blocks,
+                                    const int32_t* start_pos, int32_t n_seqs, int32_t n_new,
+                                    int32_t max_seq_len, const void* q_bf16, int32_t n_q_heads,
+                                    float scale, void* out, int32_t out_dtype, void* stream);
 
 /* Canonical codes of every pool block, indexed by (physical block * 16 + t). */
 int fmkv_pool_read_codes(const fmkv_pool* pool, void* codes, void* meta, void* stream);

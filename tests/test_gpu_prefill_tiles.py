@@ -253,3 +253,42 @@ def test_prefill_grids(gpu, ora, mode, bits, D, prefix, n, wide):
     rows = sorted({*range(min(n, 9)), *range(max(0, n - 9), n), n // 2})
     err = np.abs(out[rows] - oc.prefill(k[prefix:], v[prefix:], q, scale, rows=rows))
     assert err.max() < (2e-2 if mode == 1 else 4e-3) and err.mean() < 1.2e-4, f"{err.max():.2e} {err.mean():.2e}"
+
+
+@pytest.mark.parametrize("mode,bits,D", [(0, 4, 128), (1, 3, 256), (2, 16, 128), (0, 8, 512)])
+@pytest.mark.parametrize("n", [3, 100])
+def test_prefill_longest_length_given(gpu, ora, mode, bits, D, n):
+    """max_seq_len on a wide table: the bits of the call on a table of that
+    width; far too small or too large ones: the oracle's result all the same."""
+    import torch
+
+    starts, Hkv, Hq = [600, 40, 0, 1500], 1, 4
+    need = [(p + n + 15) // 16 for p in starts]
+    wide = torch.zeros((4, 2000), dtype=torch.int32, device="cuda")
+    pool = gpu.PagedPool(gpu.make_desc(Hkv, D, bits, mode=mode), sum(need))
+    start = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    k, v = kv_batch(n, 4 * n, Hkv, D).reshape(4, n, Hkv, D), kv_batch(n + 1, 4 * n, Hkv, D).reshape(4, n, Hkv, D)
+    q = soft_q(n, 4 * n, Hq, D).reshape(4, n, Hq, D)
+    scale, want, at = 0.3 / np.sqrt(D), [], 0
+    for s, p in enumerate(starts):
+        wide[s, :need[s]] = torch.arange(at, at + need[s], dtype=torch.int32, device="cuda")
+        at += need[s]
+        oc = ora.OracleCache(Hkv, D, bits, 0, p + n, mode=mode)
+        if p:
+            k0, v0 = kv_batch(50 + s, p, Hkv, D), kv_batch(60 + s, p, Hkv, D)
+            oc.append(k0, v0)
+            pool.append(dev_bf16(k0)[None], dev_bf16(v0)[None], wide[s:s + 1], start[2:3])
+        want.append(oc.prefill(k[s], v[s], q[s], scale))
+    want, args = np.stack(want), [dev_bf16(x) for x in (k, v, q)]
+
+    def call(table, longest):
+        return pool.prefill_step(args[0], args[1], table, start, args[2], scale, dtype=torch.float32,
+                                 max_seq_len=longest)
+
+    exact = call(wide[:, :max(need)].contiguous(), 0)
+    assert torch.equal(exact, call(wide, max(starts) + n))
+    for longest in (0, 1, 300, 32000, 1 << 30):
+        err = np.abs(call(wide, longest).cpu().numpy().astype(np.float64) - want)
+        assert err.max() < (2e-2 if mode == 1 else 4e-3) and err.mean() < 1.2e-4, f"{longest}: {err.max():.2e}"
+    with pytest.raises(gpu.Exception_):
+        call(wide, -1)
