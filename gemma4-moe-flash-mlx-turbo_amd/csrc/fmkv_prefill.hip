@@ -1100,10 +1100,10 @@ void prefill_attn_kernel(PrefillArgs a) {
   keep_own();
   load_k(nxt);
   lds_barrier();
-  // an interval between two barriers: QK of step i + 1 (past the end: of the
-  // last blocks, for nothing), softmax of step i, PV of step i - 1
+  // an interval between two barriers: QK of step i + 1, softmax of step i, PV of
+  // step i - 1; the last one has no QK (a tenth of a call of one or two steps)
 #pragma unroll 1
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < n - 1; i++) {
     fresh_offsets();
     rescale((i - 1) & 1);
     qk((i + 1) & 1);
@@ -1116,6 +1116,11 @@ void prefill_attn_kernel(PrefillArgs a) {
     lds_barrier();
     advance(i + 1);
   }
+  rescale((n - 2) & 1);
+  softmax((n - 1) & 1, s_begin + n - 1, mine, f_cur);
+  if (n > 1) pv((n - 2) & 1, std::false_type{});
+  load_v(cur);
+  lds_barrier();
   rescale((n - 1) & 1);
   pv((n - 1) & 1, std::false_type{});
 
@@ -1340,12 +1345,14 @@ size_t prefill_scratch_bytes(int cus) {
 // of LDS allow no more.
 //
 // min_split: shorter sequences stay one range, and a call without longer ones
-// has no merge launch (about 4 us, also where it finds nothing to merge):
-// 107@50, 512: 46 one range, 51 two. A grid that fills part of the chip has
-// less to gain: 4 x 300@200, 128: 46 one range, 56 three each; but 512, whose
-// work-groups have a CU each: 400@0 (100, 14 steps): 62 two ranges, 66 one; and
-// where the bound is long, the merge launch being there anyway (a wide table's
-// 2 x 150@100, 256: 47 two ranges, 53 one).
+// has no merge launch (about 4 us, also where it finds nothing to merge). At
+// 107@50 (7 steps), 512: 46 one range, 51 two. Eight waves a work-group at 128
+// and 256 need 9 steps that an average row sees: 400@0 (8 of 14), 128: 38 one
+// range, 42 two; 8 x 40@276..483 (10 to 16), 128: 53 and 38; and more where
+// the grid fills part of the chip: 4 x 300@200 (160 work-groups, 13 of 17),
+// 128: 46 one range, 56 three each. From 8 steps on gain 512 (400@0: 66 one, 62
+// two), fewer waves (256, 600@10: 75 and 60) and calls with a long bound, where
+// the merge is launched anyway (a wide table's 2 x 150@100, 256: 53 and 47).
 size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) {
   const int D = a.new_st.layout.head_dim, qp = kPfRows / a.group;
   const int64_t wgs = (int64_t)((a.n_q + qp - 1) / qp) * a.new_st.n_kv_heads;  // per unit
@@ -1355,7 +1362,10 @@ size_t prefill_plan(PrefillArgs& a, int cus, int64_t max_steps, bool may_split) 
   a.units = 0;
   a.share_rows = D < 512 && total <= (!few ? cus / 4 : D == 128 ? cus : cus / 2);
   const int64_t places = prefill_places(D, a.share_rows, cus);
-  a.min_split = D == 512 || (total <= cus && !(few && a.share_rows)) ? 8 : (int)(12 + 16 * total / cus);
+  const int mean = a.n_q / (2 * kPfKeys);  // steps that a row has less than the last, on average
+  a.min_split = D == 512 || (total <= cus && !(few && a.share_rows)) ? 8
+                : total <= cus / 4                                   ? 9 + mean
+                                                                     : (int)(5 + 16 * total / cus) + mean;
   if (!may_split || max_steps < a.min_split) return 0;
   int64_t units = places / wgs;
   const int64_t most = a.n_seqs * ((max_steps + kPfMinSteps - 1) / kPfMinSteps);
