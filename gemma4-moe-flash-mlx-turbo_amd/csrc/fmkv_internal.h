@@ -153,7 +153,7 @@ struct PrefillArgs {
   float c;            // 1/sqrt(D)
   void* out;          // [n_q][n_q_heads][D]
   int32_t out_f32;
-  // Split over the keys: grid z counts units (prefill_units) and the ranges'
+  // Split over the keys: grid z counts units (prefill_plan) and the ranges'
   // partial rows go to part_o [units][n_kv_heads][tiles][64][D] and part_ml
   // [..][64][2] for a merge; 0: one work-group per (tile, KV head, sequence).
   int32_t units = 0;
